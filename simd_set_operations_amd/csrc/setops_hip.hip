@@ -89,6 +89,7 @@ static_assert(pad_for(kNTM * 12, kMaxSeg) >= 12 && pad_for(kNTM * 20, kMaxSeg) >
 constexpr int kCapB = 3072;  // search policy: larger windows staged up to this many words
 
 constexpr uint32_t kOneScanGroups = 8;      // pair-unit scans of up to this many groups run as one workgroup
+constexpr uint32_t kOneScanParts = 32;      // ... on at most this many workgroups, each with all the sizes
 constexpr uint32_t kScanDirectGroups = 64;  // tile-count scans of up to this many groups run as one kernel
 constexpr uint64_t kMaxGrid = 1u << 22;  // grid-stride beyond this many workgroups
 constexpr int kPlaceNT = 64;   // lanes of a placement workgroup (one tile each)
@@ -461,6 +462,8 @@ int launch_units_scan(setops_hip_batch *h, const TileOut &out, hipStream_t strea
     // up to kOneScanGroups groups of pairs (serving steps, small gather batches such as the skewed
     // workload's 4,096 pairs): the scan is one workgroup, a group at a time
     const bool one = ng <= kOneScanGroups;
+    // (each workgroup scans the batch itself and writes its share of the pairs and tiles)
+    const uint32_t parts = grid_for(std::max<uint64_t>(h->P, h->plan.ntiles), kScanGroup);
     if (!one) {
         hipLaunchKernelGGL((units_reduce_kernel<kScanGroup>), dim3(ng), dim3(kScanGroup), 0, stream, h->in,
                            h->plan, 0u);
@@ -469,8 +472,12 @@ int launch_units_scan(setops_hip_batch *h, const TileOut &out, hipStream_t strea
                            h->plan.gsum2, (uint64_t)ng, 0, h->d_tot);
         HIP_TRY(hipGetLastError());
     }
-    hipLaunchKernelGGL((units_scan_kernel<kScanGroup, kOneScanGroups>), dim3(one ? 1 : ng), dim3(kScanGroup), 0, stream,
-                       h->in, h->plan, out, one ? 1 : 0);
+    if (one)
+        hipLaunchKernelGGL((units_scan_kernel<kScanGroup, kOneScanGroups>), dim3(std::min(parts, kOneScanParts)),
+                           dim3(kScanGroup), 0, stream, h->in, h->plan, out, 1);
+    else
+        hipLaunchKernelGGL((units_scan_kernel<kScanGroup, 1>), dim3(ng), dim3(kScanGroup), 0, stream, h->in, h->plan,
+                           out, 0);
     HIP_TRY(hipGetLastError());
     return SETOPS_OK;
 }
@@ -592,9 +599,9 @@ void launch_tiles_b(setops_hip_batch *h, const TileOut &out, hipStream_t stream)
 int batch_enqueue(setops_hip_batch *h, const TileOut &out, bool count_only, hipStream_t stream,
                   std::pair<hipEvent_t, hipEvent_t> *ev)
 {
-    // plan: unit prefix and tile maps, then tile starts (one pair over several merge tiles: both
-    // in one launch; one pair in one tile: none, the tile kernel takes the pair as it is)
-    const bool single_split = h->plan.single && !h->plan.direct && h->plan.policy == POLICY_MERGE;
+    // plan: unit prefix and tile maps, then tile starts (one pair over several tiles: both in one
+    // launch; one pair in one tile: none, the tile kernel takes the pair as it is)
+    const bool single_split = h->plan.single && !h->plan.direct;
     if (h->plan.direct) {
         // no plan launch
     } else if (single_split) {

@@ -130,27 +130,45 @@ __device__ __forceinline__ uint64_t pair_units(const PairBatch &in, uint32_t pol
     return (policy == POLICY_SEARCH ? (na < nb ? na : nb) : na + nb) + c0;
 }
 
-// Records, for the pair owning units [u, un), the tiles it starts and ends.
-// Search policy: a tile starting inside the pair starts at probe min(t*U - u, probes) of it (the
-// split needs no search), recorded here too, so the split kernel does not run for such batches.
-__device__ __forceinline__ void map_tiles(const TilePlan &plan, uint64_t p, uint64_t u, uint64_t un)
+// floor(u / U) for u < 2^53: the estimate by the reciprocal is off by one at most.
+__device__ __forceinline__ uint64_t tile_of_unit(uint64_t u, uint32_t U, double inv)
 {
-    const uint64_t U = plan.U;
-    const uint64_t own = un - u - plan.c0;  // the pair's probes (search policy)
-    for (uint64_t t = (u + U - 1) / U; t * U < un && t < plan.ntiles; t++) {
-        plan.tile_first[t] = (uint32_t)p;
-        if (plan.policy == POLICY_SEARCH) {
-            const uint64_t rel = t * U - u;
-            plan.tile_sa[t] = (uint32_t)(rel < own ? rel : own);
-            plan.tile_sb[t] = 0;
-        }
+    uint64_t q = (uint64_t)((double)u * inv);
+    const int64_t r = (int64_t)(u - q * U);
+    if (r < 0) q--;
+    else if (r >= (int64_t)U) q++;
+    return q;
+}
+
+// Merge policy: records, for the pair owning units [u, un) (`valid`; every lane of the wave calls,
+// with or without a pair), the tiles it starts and ends: the tiles t whose first unit tU lies in it
+// and the tiles whose last unit does.  A lane writes up to kMapOwn tiles of each kind itself; the tiles
+// of longer pairs are written by the whole wave, 64 at a time, one pair after another.
+constexpr uint32_t kMapOwn = 2;
+__device__ __forceinline__ void map_tiles(const TilePlan &plan, bool valid, uint32_t p, uint64_t u, uint64_t un)
+{
+    const uint32_t U = plan.U;
+    const double inv = 1.0 / (double)U;
+    uint32_t f0 = 0, f1 = 0, l0 = 0, l1 = 0;
+    if (valid && un > u) {
+        const uint64_t q0 = tile_of_unit(u, U, inv), q1 = tile_of_unit(un, U, inv);
+        const uint64_t nt = plan.ntiles;
+        f0 = (uint32_t)min(q0 + (u > q0 * U ? 1u : 0u), nt);
+        f1 = (uint32_t)min(q1 + (un > q1 * U ? 1u : 0u), nt);
+        l0 = (uint32_t)min(q0, nt);
+        l1 = (uint32_t)(un >= plan.utotal ? nt : min(q1, nt));  // the last tile ends with the last unit
     }
-    for (uint64_t t = u / U; t < plan.ntiles; t++) {
-        uint64_t last = (t + 1) * U;
-        if (last > plan.utotal) last = plan.utotal;
-        last -= 1;
-        if (last >= un) break;
-        if (last >= u) plan.tile_last[t] = (uint32_t)p;
+    const bool big = f1 - f0 > kMapOwn || l1 - l0 > kMapOwn;
+    if (!big) {
+        for (uint32_t t = f0; t < f1; t++) plan.tile_first[t] = p;
+        for (uint32_t t = l0; t < l1; t++) plan.tile_last[t] = p;
+    }
+    for (uint64_t m = ballot(big); m; m &= m - 1) {
+        const int l = __builtin_ctzll(m);
+        auto rl = [&](uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane((int)v, l); };
+        const uint32_t bp = rl(p), bf0 = rl(f0), bf1 = rl(f1), bl0 = rl(l0), bl1 = rl(l1);
+        for (uint32_t t = bf0 + lane_id(); t < bf1; t += kWave) plan.tile_first[t] = bp;
+        for (uint32_t t = bl0 + lane_id(); t < bl1; t += kWave) plan.tile_last[t] = bp;
     }
 }
 
@@ -163,48 +181,25 @@ __device__ __forceinline__ void plan_reset(const TileOut &out)
     if (out.error) *out.error = 0;
 }
 
-// CSR batches: unit prefix in closed form, tile maps, zeroed per-pair counts.  Grid-stride over
-// pairs.  In single-pair mode it also writes the pair's offsets.
+// CSR batches, merge policy: unit prefix in closed form, tile maps, zeroed per-pair counts.
+// Grid-stride over pairs.
 __global__ void plan_csr_kernel(PairBatch in, TilePlan plan, TileOut out)
 {
     const uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const uint64_t gsz = (uint64_t)gridDim.x * blockDim.x;
-    auto abeg = [&](uint64_t p) -> uint64_t { return plan.single ? 0 : in.a_beg[p]; };
-    auto bbeg = [&](uint64_t p) -> uint64_t { return plan.single ? 0 : in.b_beg[p]; };
-    auto aend = [&](uint64_t p) -> uint64_t { return plan.single ? plan.single_na : in.a_end[p]; };
-    auto bend = [&](uint64_t p) -> uint64_t { return plan.single ? plan.single_nb : in.b_end[p]; };
-    if (plan.single && gid == 0) {
-        plan.single_off[0] = 0;
-        plan.single_off[1] = plan.single_na;
-        plan.single_off[2] = 0;
-        plan.single_off[3] = plan.single_nb;
-        if (plan.direct) {
-            // the one tile starts at the pair's start (the split of unit 0); its runs are the sets
-            plan.tile_sa[0] = 0;
-            plan.tile_sb[0] = 0;
-            plan.tile_ga[0] = 0;
-            plan.tile_ga[1] = plan.single_na;
-            plan.tile_gb[0] = 0;
-            plan.tile_gb[1] = plan.single_nb;
+    const uint64_t a0 = in.a_beg[0], b0 = in.b_beg[0];
+    for (uint64_t pw = gid - lane_id(); pw < in.P; pw += gsz) {  // the wave's first pair (uniform)
+        const uint64_t p = pw + lane_id();
+        const bool valid = p < in.P;
+        uint64_t u = 0, un = 0;
+        if (valid) {
+            u = in.a_beg[p] - a0 + in.b_beg[p] - b0 + (uint64_t)plan.c0 * p;
+            un = in.a_end[p] - a0 + in.b_end[p] - b0 + (uint64_t)plan.c0 * (p + 1);
+            plan.uoff[p] = u;
+            if (p + 1 == in.P) plan.uoff[in.P] = un;
+            if (out.counts) out.counts[p] = 0;
         }
-    }
-    const uint64_t a0 = abeg(0), b0 = bbeg(0);
-    for (uint64_t p = gid; p < in.P; p += gsz) {
-        const uint64_t ab = abeg(p) - a0, bb = bbeg(p) - b0;
-        const uint64_t ae = aend(p) - a0, be = bend(p) - b0;
-        uint64_t u, un;
-        if (plan.policy == POLICY_SEARCH) {
-            // min() does not telescope: only single-pair plans take this branch
-            u = 0;
-            un = ((ae - ab) < (be - bb) ? (ae - ab) : (be - bb)) + plan.c0;
-        } else {
-            u = ab + bb + (uint64_t)plan.c0 * p;
-            un = ae + be + (uint64_t)plan.c0 * (p + 1);
-        }
-        plan.uoff[p] = u;
-        if (p + 1 == in.P) plan.uoff[in.P] = un;
-        map_tiles(plan, p, u, un);
-        if (out.counts) out.counts[p] = 0;
+        map_tiles(plan, valid, (uint32_t)p, u, un);
     }
     if (gid == 0) plan_reset(out);
 }
@@ -293,23 +288,29 @@ __global__ __launch_bounds__(NT) void groups_scan_kernel(unsigned long long *gsu
 }
 
 // Per-group scan of pair units plus the group base: uoff, tile maps, zeroed counts.  With
-// `one_group` (a batch of at most NT * MAXCHUNK pairs) one workgroup scans the whole batch, the
-// base is 0 and the group-sum kernels do not run.
+// `one_group` (a batch of at most NT * MAXCHUNK pairs) the base is 0, the group-sum kernels do not
+// run, and every workgroup scans the whole batch itself and writes its share of the pairs and tiles.
+// The pairs' starts stay in LDS, where each tile finds the pairs of its first and last unit by binary
+// search, a tile per thread: the same work for every tile however its pairs are sized.  (3,000
+// skewed pairs over 15,600 search tiles: 78 us when the threads that scan the pairs write their tiles,
+// in one workgroup, 30 us when a wave writes a pair's tiles together, 7 us here.)
 template <int NT, int MAXCHUNK>
 __global__ __launch_bounds__(NT) void units_scan_kernel(PairBatch in, TilePlan plan, TileOut out, int one_group)
 {
     static_assert(NT == (int)kScanGroup, "one thread per pair of a group");
     __shared__ unsigned long long wsum[NT / kWave];
-    // one_group: a single workgroup scans all pairs, thread t the C = ceil(P / NT) <= MAXCHUNK
-    // consecutive pairs from t*C (their sizes load together, one block scan of the thread sums);
-    // otherwise group blockIdx.x, one pair per thread, after the group sums' scan
-    const uint32_t C = one_group ? (uint32_t)((in.P + NT - 1) / NT) : 1u;
-    const uint64_t p0 = one_group ? (uint64_t)threadIdx.x * C : (uint64_t)blockIdx.x * kScanGroup + threadIdx.x;
+    __shared__ unsigned long long start[NT * MAXCHUNK + 1];
+    // the pairs scanned: [pb, pb + n), thread t the C consecutive ones from t * C (their sizes load
+    // together, one block scan of the thread sums)
+    const uint64_t pb = one_group ? 0 : (uint64_t)blockIdx.x * kScanGroup;
+    const uint32_t n = (uint32_t)(one_group ? in.P : min((uint64_t)kScanGroup, in.P - pb));
+    const uint32_t C = one_group ? (n + NT - 1) / NT : 1u;
+    const uint32_t i0 = threadIdx.x * C;
     unsigned long long vs[MAXCHUNK], local = 0;
 #pragma unroll
     for (int c = 0; c < MAXCHUNK; c++) {
-        const uint64_t p = p0 + (uint64_t)c;
-        vs[c] = ((uint32_t)c < C && p < in.P) ? pair_units(in, plan.policy, plan.c0, p) : 0ull;
+        const uint32_t i = i0 + (uint32_t)c;
+        vs[c] = ((uint32_t)c < C && i < n) ? pair_units(in, plan.policy, plan.c0, pb + i) : 0ull;
         local += vs[c];
     }
     // 64-bit block scan of the thread sums: wave scan, then wave totals
@@ -327,22 +328,60 @@ __global__ __launch_bounds__(NT) void units_scan_kernel(PairBatch in, TilePlan p
     u += x - local;  // the thread's first pair starts here
 #pragma unroll
     for (int c = 0; c < MAXCHUNK; c++) {
-        const uint64_t p = p0 + (uint64_t)c;
-        if ((uint32_t)c < C && p < in.P) {
-            const uint64_t un = u + vs[c];
-            plan.uoff[p] = u;
-            if (p + 1 == in.P) plan.uoff[in.P] = un;
-            map_tiles(plan, p, u, un);
-            if (out.counts) out.counts[p] = 0;
-            u = un;
+        const uint32_t i = i0 + (uint32_t)c;
+        if ((uint32_t)c < C && i < n) {
+            start[i] = u;
+            u += vs[c];
+            if (i + 1 == n) start[n] = u;
         }
+    }
+    __syncthreads();
+    const uint32_t part = one_group ? blockIdx.x : 0u, parts = one_group ? gridDim.x : 1u;
+    for (uint32_t i = part * NT + threadIdx.x; i < n; i += parts * NT) {
+        plan.uoff[pb + i] = start[i];
+        if (out.counts) out.counts[pb + i] = 0;
+    }
+    const bool last = one_group ? part == 0 : pb + n == in.P;
+    if (last && threadIdx.x == 0) plan.uoff[in.P] = start[n];
+    // the last pair that starts at or before unit v (v >= start[0]; n if the pairs end at or before it)
+    auto owner = [&](unsigned long long v) {
+        uint32_t lo = 0, hi = n + 1;
+        while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (start[mid] <= v) lo = mid; else hi = mid;
+        }
+        return lo;
+    };
+    // tiles: all of them in shares, or those whose first unit (last unit) lies in the group's pairs
+    const uint32_t U = plan.U;
+    uint32_t tb = 0, te = plan.ntiles;
+    if (!one_group) {
+        const double inv = 1.0 / (double)U;
+        tb = (uint32_t)min(tile_of_unit(start[0], U, inv), (uint64_t)plan.ntiles);
+        te = pb + n == in.P ? plan.ntiles : (uint32_t)min(tile_of_unit(start[n], U, inv) + 1, (uint64_t)plan.ntiles);
+    }
+    for (uint32_t t = tb + part * NT + threadIdx.x; t < te; t += parts * NT) {
+        const unsigned long long v0 = (unsigned long long)t * U;
+        const unsigned long long v1 = min(v0 + U, (unsigned long long)plan.utotal) - 1;
+        if (v0 >= start[0] && (v0 < start[n] || last)) {
+            const uint32_t p = owner(v0);
+            plan.tile_first[t] = (uint32_t)(pb + p);
+            if (plan.policy == POLICY_SEARCH) {
+                // the tile starts at probe min(t U - the pair's start, probes) of its first pair (the
+                // split needs no search, so the split kernel does not run for such batches)
+                const unsigned long long rel = v0 - start[p], own = p < n ? start[p + 1] - start[p] - plan.c0 : 0ull;
+                plan.tile_sa[t] = (uint32_t)min(rel, own);
+                plan.tile_sb[t] = 0;
+            }
+        }
+        if (v1 >= start[0] && (v1 < start[n] || last)) plan.tile_last[t] = (uint32_t)(pb + owner(v1));
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) plan_reset(out);
 }
 
-// One pair over several tiles (single mode, merge policy): the plan and the split in one launch.
-// Pair 0 owns units [0, na + nb + c0) -- every tile lies in it -- so thread t writes tile t's maps
-// and finds its merge-path split of unit t*U directly (the search of plan_split_kernel).
+// One pair over several tiles (single mode): the plan and the split in one launch.  Pair 0 owns all
+// the units -- every tile lies in it -- so thread t writes tile t's maps and finds where it starts:
+// its merge-path split of unit t*U (the search of plan_split_kernel), or its first probe.
 __global__ void plan_split_single_kernel(PairBatch in, TilePlan plan, TileOut out)
 {
     const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -353,7 +392,7 @@ __global__ void plan_split_single_kernel(PairBatch in, TilePlan plan, TileOut ou
         plan.single_off[2] = 0;
         plan.single_off[3] = nb;
         plan.uoff[0] = 0;
-        plan.uoff[1] = na + nb + plan.c0;
+        plan.uoff[1] = (plan.policy == POLICY_SEARCH ? min(na, nb) : na + nb) + plan.c0;
         plan.tile_ga[plan.ntiles] = na;
         plan.tile_gb[plan.ntiles] = nb;
         if (out.counts) out.counts[0] = 0;
@@ -363,6 +402,11 @@ __global__ void plan_split_single_kernel(PairBatch in, TilePlan plan, TileOut ou
     plan.tile_first[t] = 0;
     plan.tile_last[t] = 0;
     const uint64_t rel = t * plan.U;
+    if (plan.policy == POLICY_SEARCH) {
+        plan.tile_sa[t] = (uint32_t)min(rel, min(na, nb));
+        plan.tile_sb[t] = 0;
+        return;
+    }
     const uint64_t d = rel < na + nb ? rel : na + nb;
     uint64_t lo = d > nb ? d - nb : 0, hi = d < na ? d : na;
     const uint32_t *__restrict__ A = in.A;
