@@ -31,9 +31,9 @@ DOMINANT_KERNEL = {
     "hip_branchless_merge": "setops::merge_tile_kernel<256, 20, 130, false, false, false, 0, false>",
     "hip_shuffling": "setops::merge_tile_kernel<256, 20, 130, false, false, false, 1, false>",
     "hip_qfilter": "setops::merge_tile_kernel<256, 20, 130, false, false, false, 2, false>",
-    "hip_galloping": "setops::search_tile_kernel<256, 2, 130, 3072, false, false, 1, false>",
-    "hip_binary_search": "setops::search_tile_kernel<256, 2, 130, 3072, false, false, 0, false>",
-    "hip_simd_galloping": "setops::search_tile_kernel<256, 2, 130, 3072, false, false, 2, false>",
+    "hip_galloping": "setops::search_tile_kernel<256, 2, 130, 3584, false, false, 1, false>",
+    "hip_binary_search": "setops::search_tile_kernel<256, 2, 130, 3584, false, false, 0, false>",
+    "hip_simd_galloping": "setops::search_tile_kernel<256, 2, 130, 3584, false, false, 2, false>",
 }
 
 

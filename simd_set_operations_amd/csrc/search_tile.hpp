@@ -6,12 +6,13 @@
 // U = NT*KS probes whatever the sizes of the larger sets.  Per tile:
 //   1. segment table; stage the probe windows in LDS (the smaller side of each pair, which may
 //      be A or B -- orientation does not change the result, A∩B ascending),
-//   2. narrow each pair's larger set to [lo, hi): lower bound of the segment's first probe and
-//      upper bound of its last probe, by a wave-cooperative 64-way partition search,
-//   3. stage the narrowed larger windows in LDS while they fit (a prefix of the segments); the
-//      rest are searched in global memory,
-//   4. each lane looks up its KS probes, in order, from where the previous probe landed:
-//      galloping (exponential then binary, galloping.rs:7-30), binary search over the rest of
+//   2. narrow the larger set of a pair that other tiles share to [lo, hi): lower bound of the
+//      segment's first probe and upper bound of its last probe, by a wave-cooperative 64-way
+//      partition search,
+//   3. stage the larger windows in LDS, whole where they are short, else the first element of every
+//      m-th line, while they fit (a prefix of the segments); the rest are searched in global memory,
+//   4. each lane looks up its KS probes, in sampled windows by groups of lanes that read the line
+//      found, in staged and unstaged ones in order, from where the previous probe landed: galloping (exponential then binary, galloping.rs:7-30), binary search over the rest of
 //      the window (binary_search_intersect, galloping.rs:32-49) or block galloping with a full
 //      compare of the last block (simd_galloping.rs:49-107),
 //   5. block scan of hits, results (probe values; BSR: base and state AND) staged in order,
@@ -36,8 +37,11 @@ struct SearchSmem {
     uint32_t seg_wa[MAXSEG];            // probes in the window
     uint32_t seg_lo[MAXSEG];            // narrowed larger window [lo, hi), pair-relative
     uint32_t seg_hi[MAXSEG];
-    uint32_t seg_lb[MAXSEG];            // LDS index of lkey[lo], or kNotStaged
-    uint32_t seg_flags[MAXSEG];         // bit0: pair starts here, bit1: ends here, bit2: larger side is A
+    uint32_t seg_lb[MAXSEG];            // LDS index of lkey[lo] (or of its samples), or kNotStaged
+    uint32_t seg_m[MAXSEG];             // lines per sample of a sampled window, 0: staged whole
+    // bit0: pair starts here, bit1: ends here, bit2: larger side is A; from bit 8: samples
+    uint32_t seg_flags[MAXSEG];
+    uint32_t narrow[4];                 // first segment's narrowed window, last segment's
     uint64_t seg_lbase[MAXSEG];         // pool index of the larger set's first element
     uint32_t lane_mask[NT];
     uint32_t lane_pfx[NT];
@@ -82,7 +86,6 @@ __device__ __forceinline__ uint32_t lower_bound_from(const Arr &arr, uint32_t lo
 // Search modes of the probes: binary search, galloping, or galloping over blocks with a full
 // compare of the last block (simd_galloping).
 enum : int { SM_BINARY = 0, SM_GALLOP = 1, SM_BLOCK = 2 };
-constexpr uint32_t kBlockLds = 8;    // block of a staged (LDS) window: 8 reads
 constexpr uint32_t kBlockPool = 32;  // block of a pool window: one 128-byte span, nine 16-byte loads
 
 // Blocks [lo + W b, lo + W b + W) of arr[lo, hi): the first block whose last element is >= x, found
@@ -110,24 +113,10 @@ __device__ __forceinline__ uint32_t gallop_blocks(const Arr &arr, uint32_t lo, u
     return bl;
 }
 
-// Lower bound of x in arr[lo, hi) by block galloping; the block that can hold x is counted in
-// full, W independent reads in place of the last log2(W) dependent steps (block_compare,
-// simd_galloping.rs:272-296).  For LDS arrays.
-template <uint32_t W, class Arr>
-__device__ __forceinline__ uint32_t lower_bound_block(const Arr &arr, uint32_t lo, uint32_t hi, uint32_t x)
-{
-    const uint32_t b = gallop_blocks<W>(arr, lo, hi, x);
-    const uint32_t s0 = lo + W * b;
-    if (s0 >= hi) return hi;
-    const uint32_t n = (hi - s0 < W) ? hi - s0 : W;
-    uint32_t lt = 0;
-#pragma unroll
-    for (uint32_t j = 0; j < W; j++) lt += (j < n && arr(s0 + j) < x) ? 1u : 0u;
-    return s0 + lt;
-}
-
-// lower_bound_block over a window of a resident pool, L = P + g, P readable up to pool elements
-// and 16-byte aligned: the last block is read as the aligned 16-byte chunks that cover it (one
+// Lower bound of x in L[lo, hi) by block galloping over a window of a resident pool, L = P + g, P
+// readable up to pool elements and 16-byte aligned; the block that can hold x is counted in full
+// (block_compare, simd_galloping.rs:272-296), W independent reads in place of the last log2(W)
+// dependent steps: the last block is read as the aligned 16-byte chunks that cover it (one
 // round trip).  Also reports whether the window holds x.  Pool values are compared XOR f (x is
 // already in that space).
 __device__ __forceinline__ uint32_t lower_bound_block_pool(const uint32_t *__restrict__ P, uint64_t pool, uint64_t g,
@@ -254,32 +243,43 @@ __device__ __forceinline__ uint32_t lane_perm(uint32_t v, uint32_t src)
     return (uint32_t)__builtin_amdgcn_ds_bpermute((int)(src << 2), (int)v);
 }
 
-// For the NP probes of every lane (probe k of lane p: window blk[k], lh[k], x[k]): entries <= x among
-// positions [lo, hi) of the 16-entry block blk of arr (entries 16 blk .. 16 blk + 15, arr holding
-// n entries); lh = lo | hi << 8, 0 for no window.  Round r serves probe k = r / 4 of lanes
-// 16 (r % 4) .. 16 (r % 4) + 15, one per group of 4 lanes; all 4 NP loads are in flight together.
-template <int NP>
-__device__ __forceinline__ void coop_count16(const uint32_t *__restrict__ arr, uint64_t n, const uint32_t (&blk)[NP],
-                                             const uint32_t (&lh)[NP], const uint32_t (&x)[NP], uint32_t (&res)[NP])
+// The value of the lane 1 or 2 away in its group of four (xor), and of lane 7 - i of its eight, by DPP.
+__device__ __forceinline__ uint32_t quad_xor1(uint32_t v)
 {
-    constexpr int R = 4 * NP;
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, false);
+}
+__device__ __forceinline__ uint32_t quad_xor2(uint32_t v)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xf, 0xf, false);
+}
+__device__ __forceinline__ uint32_t half_mirror(uint32_t v)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, false);
+}
+
+// For the probe x of every lane: entries <= x among positions [lo, hi) of the 16-entry block blk of
+// arr (entries 16 blk .. 16 blk + 15, arr holding n entries); lh = lo | hi << 8, 0 for no window.
+// Round r serves lanes 16 r .. 16 r + 15, one per group of 4 lanes; all four loads are in flight
+// together.
+__device__ __forceinline__ uint32_t coop_count16(const uint32_t *__restrict__ arr, uint64_t n, uint32_t blk, uint32_t lh,
+                                                 uint32_t x)
+{
     const uint32_t lane = lane_id();
     const uint32_t c = lane & 3u;  // the chunk this lane reads of the block it serves
-    uint4 v[R];
-    uint32_t plh[R];
+    uint4 v[4];
+    uint32_t plh[4];
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-        const uint32_t p = 16u * (uint32_t)(r & 3) + (lane >> 2);  // the lane whose probe r / 4 is served
-        const uint32_t pb = lane_perm(blk[r >> 2], p);
-        plh[r] = lane_perm(lh[r >> 2], p);
+    for (int r = 0; r < 4; r++) {
+        const uint32_t p = 16u * (uint32_t)r + (lane >> 2);  // the lane whose probe is served
+        const uint32_t pb = lane_perm(blk, p);
+        plh[r] = lane_perm(lh, p);
         v[r] = plh[r] ? load_chunk(arr, n, 16ull * pb + 4u * c) : make_uint4(0u, 0u, 0u, 0u);
     }
+    uint32_t res = 0;
 #pragma unroll
-    for (int k = 0; k < NP; k++) res[k] = 0;
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        const uint32_t p = 16u * (uint32_t)(r & 3) + (lane >> 2);
-        const uint32_t px = lane_perm(x[r >> 2], p);
+    for (int r = 0; r < 4; r++) {
+        const uint32_t p = 16u * (uint32_t)r + (lane >> 2);
+        const uint32_t px = lane_perm(x, p);
         const uint32_t lo = plh[r] & 0xFFu, hi = plh[r] >> 8;
         const uint32_t w[4] = {v[r].x, v[r].y, v[r].z, v[r].w};
         uint32_t k = 0;
@@ -288,133 +288,117 @@ __device__ __forceinline__ void coop_count16(const uint32_t *__restrict__ arr, u
             const uint32_t e = 4u * c + j;
             k += (e >= lo && e < hi && w[j] <= px) ? 1u : 0u;
         }
-        k += __shfl_xor(k, 1, kWave);
-        k += __shfl_xor(k, 2, kWave);
-        const uint32_t t = lane_perm(k, 4u * (lane & 15u));  // lane 16 (r % 4) + i reads group i
-        if ((lane >> 4) == (uint32_t)(r & 3)) res[r >> 2] = t;
+        k += quad_xor1(k);
+        k += quad_xor2(k);
+        const uint32_t t = lane_perm(k, 4u * (lane & 15u));  // lane 16 r + i reads group i
+        if ((lane >> 4) == (uint32_t)r) res = t;
     }
+    return res;
 }
 
-// For the NP probes of every lane: the position of x (compared XOR f) among positions [lo, hi) of
-// the 32-element line `line` of B (elements 32 line .. 32 line + 31), or 32 when absent; lh as
-// above.  Round r serves probe k = r / 8 of lanes 8 (r % 8) .. 8 (r % 8) + 7, one per group of 8.
-template <int NP>
-__device__ __forceinline__ void coop_find32(const uint32_t *__restrict__ B, uint64_t pool, const uint32_t (&line)[NP],
-                                            const uint32_t (&lh)[NP], const uint32_t (&x)[NP], uint32_t f,
-                                            uint32_t (&res)[NP])
+// The positions [from, to) of a 32-element line as a mask, from <= 31, to <= 32.
+__device__ __forceinline__ uint32_t line_mask(uint32_t from, uint32_t to)
 {
-    constexpr int R = 8 * NP;
+    return to > from ? (~0u >> (32u - to)) & (~0u << from) : 0u;
+}
+
+// For the probe x of every lane (in the compare space): the position of x in the 32-element line
+// `line` of B (or of A, with AB and `a`; elements 32 line .. 32 line + 31) among the positions vm (0:
+// no probe), or 32 when absent.  Without POS only whether x is there: 0 or 32.  Round r serves
+// lanes 8 r .. 8 r + 7, one per group of 8 lanes; all eight loads are in flight together.
+template <bool POS, bool AB>
+__device__ __forceinline__ uint32_t coop_find32(const PairBatch &in, uint32_t line, uint32_t vm, bool a, uint32_t x)
+{
     const uint32_t lane = lane_id();
     const uint32_t c = lane & 7u;
-    uint4 v[R];
-    uint32_t plh[R];
+    uint4 v[8];
+    uint32_t pvm[8];
+    const uint64_t am = AB ? ballot(a) : 0ull;
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-        const uint32_t p = 8u * (uint32_t)(r & 7) + (lane >> 3);
-        const uint32_t pl = lane_perm(line[r >> 3], p);
-        plh[r] = lane_perm(lh[r >> 3], p);
-        v[r] = plh[r] ? load_chunk(B, pool, 32ull * pl + 4u * c) : make_uint4(0u, 0u, 0u, 0u);
+    for (int r = 0; r < 8; r++) {
+        const uint32_t p = 8u * (uint32_t)r + (lane >> 3);
+        const uint32_t pl = lane_perm(line, p);
+        pvm[r] = lane_perm(vm, p);
+        const bool pa = AB && ((am >> p) & 1u);
+        v[r] = pvm[r] ? load_chunk(pa ? in.A : in.B, pa ? in.a_pool : in.b_pool, 32ull * pl + 4u * c)
+                      : make_uint4(0u, 0u, 0u, 0u);
     }
+    uint32_t res = 32;
+    const uint32_t xf = x ^ in.sflip;
 #pragma unroll
-    for (int k = 0; k < NP; k++) res[k] = 32;
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        const uint32_t p = 8u * (uint32_t)(r & 7) + (lane >> 3);
-        const uint32_t px = lane_perm(x[r >> 3], p);
-        const uint32_t lo = plh[r] & 0xFFu, hi = plh[r] >> 8;
-        const uint32_t w[4] = {v[r].x ^ f, v[r].y ^ f, v[r].z ^ f, v[r].w ^ f};
-        uint32_t h = 0;  // position + 1 of the match (a set holds x at most once)
-#pragma unroll
-        for (uint32_t j = 0; j < 4; j++) {
-            const uint32_t e = 4u * c + j;
-            h = (e >= lo && e < hi && w[j] == px) ? e + 1u : h;
+    for (int r = 0; r < 8; r++) {
+        const uint32_t px = lane_perm(xf, 8u * (uint32_t)r + (lane >> 3));
+        const uint32_t eq = (v[r].x == px ? 1u : 0u) | (v[r].y == px ? 2u : 0u) | (v[r].z == px ? 4u : 0u) |
+                            (v[r].w == px ? 8u : 0u);
+        const uint32_t hit = eq & (pvm[r] >> (4u * c));  // one bit at most (a set holds x at most once)
+        if constexpr (POS) {
+            uint32_t h = hit ? 4u * c + (uint32_t)__builtin_ctz(hit) + 1u : 0u;  // position + 1
+            h |= quad_xor1(h);
+            h |= quad_xor2(h);
+            h |= half_mirror(h);  // the other four lanes of the eight
+            const uint32_t t = lane_perm(h, 8u * (lane & 7u));  // lane 8 r + i reads group i
+            if ((lane >> 3) == (uint32_t)r) res = t ? t - 1u : 32u;
+        } else {
+            // group i of round r answers lane 8 r + i
+            const uint64_t b = ballot(hit != 0);
+            if ((lane >> 3) == (uint32_t)r) res = ((b >> (8u * (lane & 7u))) & 0xFFu) ? 0u : 32u;
         }
-        h |= __shfl_xor(h, 1, kWave);
-        h |= __shfl_xor(h, 2, kWave);
-        h |= __shfl_xor(h, 4, kWave);
-        const uint32_t t = lane_perm(h, 8u * (lane & 7u));  // lane 8 (r % 8) + i reads group i
-        if ((lane >> 3) == (uint32_t)(r & 7)) res[r >> 3] = t ? t - 1u : 32u;
     }
+    return res;
 }
 
-// Pool index of x in B[g0, g1), or kNoPos, for the NP probes of every lane of the wave (on = false:
-// no probe), through the top level top[j - tj0] = B[kTopStride j] in LDS, the middle level
-// mid[m] = idx[kMidIdx m] and the index idx[k] = B[32 k] (values in the compare space), with the
-// global reads made by groups of lanes.  The windows it reads each lie in one aligned block:
-// the middle-level entries over one top-level interval are those of one 16-entry block (top
-// entries are every 16th middle entry), likewise the index entries under one middle-level
-// interval, and the candidates of B one 32-element line.
-template <int NP>
-__device__ __forceinline__ void coop_index_probe_top(const bool (&on_)[NP], const uint32_t *__restrict__ B, uint64_t pool,
-                                                     const uint32_t *__restrict__ idx, const uint32_t *__restrict__ mid,
-                                                     const uint32_t *top, uint64_t tj0, const uint64_t (&g0)[NP],
-                                                     const uint64_t (&g1)[NP], const uint32_t (&x)[NP], uint32_t f,
-                                                     uint64_t (&q)[NP])
+// Pool index of x in B[g0, g1) (without POS: any index of its line), or kNoPos, for the probe of every
+// lane of the wave (on = false: no probe), through the top level top[j - tj0] = B[kTopStride j] in
+// LDS, the middle level in.b_mid[m] = in.b_idx[kMidIdx m] and the index in.b_idx[k] = B[32 k] (values
+// in the compare space), with the global reads made by groups of lanes.  The windows it reads
+// each lie in one aligned block: the middle-level entries over one top-level interval are those of
+// one 16-entry block (top entries are every 16th middle entry), likewise the index entries under one
+// middle-level interval, and the candidates of B one 32-element line.
+template <bool POS>
+__device__ __forceinline__ uint64_t coop_index_probe_top(const PairBatch &in, bool on, const uint32_t *top, uint64_t tj0,
+                                                         uint64_t g0, uint64_t g1, uint32_t x)
 {
-    bool on[NP];
-    uint64_t L[NP], H[NP], mb[NP], me[NP];
-    uint32_t mblk[NP], mlh[NP];
-#pragma unroll
-    for (int k = 0; k < NP; k++) {
-        on[k] = on_[k] && g0[k] < g1[k];
-        L[k] = H[k] = mb[k] = me[k] = 0;
-        if (on[k]) {
-            const uint64_t kb = (g0[k] + 31) / 32, ke = (g1[k] + 31) / 32;
-            const uint64_t jb = (kb + kTopIdx - 1) / kTopIdx, je = (ke + kTopIdx - 1) / kTopIdx;
-            uint64_t lo = jb, hi = je;  // first top entry > x
-            while (lo < hi) {
-                const uint64_t m = (lo + hi) >> 1;
-                if (top[m - tj0] <= x[k]) lo = m + 1; else hi = m;
-            }
-            L[k] = (lo > jb) ? kTopIdx * (lo - 1) + 1 : kb;
-            H[k] = (lo < je) ? kTopIdx * lo : ke;
-            mb[k] = (L[k] + kMidIdx - 1) / kMidIdx;
-            me[k] = (H[k] + kMidIdx - 1) / kMidIdx;
+    on = on && g0 < g1;
+    uint64_t L = 0, H = 0, mb = 0, me = 0;
+    if (on) {
+        const uint64_t kb = (g0 + 31) / 32, ke = (g1 + 31) / 32;
+        const uint64_t jb = (kb + kTopIdx - 1) / kTopIdx, je = (ke + kTopIdx - 1) / kTopIdx;
+        uint64_t lo = jb, hi = je;  // first top entry > x
+        while (lo < hi) {
+            const uint64_t m = (lo + hi) >> 1;
+            if (top[m - tj0] <= x) lo = m + 1; else hi = m;
         }
-        // middle level: [mb, me) inside block mb / 16
-        mblk[k] = (uint32_t)(mb[k] >> 4);
-        mlh[k] = (on[k] && me[k] > mb[k]) ? (uint32_t)(mb[k] & 15u) | ((uint32_t)(me[k] - 16ull * mblk[k]) << 8) : 0u;
+        L = (lo > jb) ? kTopIdx * (lo - 1) + 1 : kb;
+        H = (lo < je) ? kTopIdx * lo : ke;
+        mb = (L + kMidIdx - 1) / kMidIdx;
+        me = (H + kMidIdx - 1) / kMidIdx;
     }
-    uint32_t mc[NP];
-    coop_count16<NP>(mid, (pool + kMidStride - 1) / kMidStride, mblk, mlh, x, mc);
-    uint64_t L2[NP];
-    uint32_t iblk[NP], ilh[NP];
-#pragma unroll
-    for (int k = 0; k < NP; k++) {
-        uint64_t H2 = 0;
-        L2[k] = 0;
-        if (on[k]) {
-            const uint64_t ms = mb[k] + mc[k];
-            L2[k] = (ms > mb[k]) ? kMidIdx * (ms - 1) + 1 : L[k];
-            H2 = (ms < me[k]) ? kMidIdx * ms : H[k];
-        }
-        // index: [L2, H2) inside block L2 / 16; the first entry > x is L2 + count
-        iblk[k] = (uint32_t)(L2[k] >> 4);
-        ilh[k] = (on[k] && H2 > L2[k]) ? (uint32_t)(L2[k] & 15u) | ((uint32_t)(H2 - 16ull * iblk[k]) << 8) : 0u;
+    // middle level: [mb, me) inside block mb / 16
+    const uint32_t mblk = (uint32_t)(mb >> 4);
+    const uint32_t mlh = (on && me > mb) ? (uint32_t)(mb & 15u) | ((uint32_t)(me - 16ull * mblk) << 8) : 0u;
+    const uint32_t mc = coop_count16(in.b_mid, (in.b_pool + kMidStride - 1) / kMidStride, mblk, mlh, x);
+    uint64_t L2 = 0, H2 = 0;
+    if (on) {
+        const uint64_t ms = mb + mc;
+        L2 = (ms > mb) ? kMidIdx * (ms - 1) + 1 : L;
+        H2 = (ms < me) ? kMidIdx * ms : H;
     }
-    uint32_t ic[NP];
-    coop_count16<NP>(idx, (pool + 31) / 32, iblk, ilh, x, ic);
-    uint32_t line[NP], blh[NP];
-    bool bon[NP];
-#pragma unroll
-    for (int k = 0; k < NP; k++) {
-        // B: the line [32(kk-1), 32 kk) holds every candidate; positions inside [g0, g1) and the pool
-        const uint64_t kk = L2[k] + ic[k];
-        bon[k] = on[k] && kk > 0;
-        const uint64_t base = bon[k] ? 32 * (kk - 1) : 0;
-        line[k] = (uint32_t)(base >> 5);
-        blh[k] = 0;
-        if (bon[k]) {
-            const uint64_t e1 = g1[k] < pool ? g1[k] : pool;
-            const uint32_t lo = g0[k] > base ? (uint32_t)min(g0[k] - base, (uint64_t)32) : 0u;
-            const uint32_t hi = e1 > base ? (uint32_t)min(e1 - base, (uint64_t)32) : 0u;
-            blh[k] = lo < hi ? lo | (hi << 8) : 0u;
-        }
+    // index: [L2, H2) inside block L2 / 16; the first entry > x is L2 + count
+    const uint32_t iblk = (uint32_t)(L2 >> 4);
+    const uint32_t ilh = (on && H2 > L2) ? (uint32_t)(L2 & 15u) | ((uint32_t)(H2 - 16ull * iblk) << 8) : 0u;
+    const uint32_t ic = coop_count16(in.b_idx, (in.b_pool + 31) / 32, iblk, ilh, x);
+    // B: the line [32(kk-1), 32 kk) holds every candidate; positions inside [g0, g1) and the pool
+    const uint64_t kk = L2 + ic;
+    const bool bon = on && kk > 0;
+    const uint64_t base = bon ? 32 * (kk - 1) : 0;
+    uint32_t vm = 0;
+    if (bon) {
+        const uint64_t e1 = min(g1, in.b_pool);
+        vm = line_mask(g0 > base ? (uint32_t)min(g0 - base, (uint64_t)31) : 0u,
+                       e1 > base && base + 32 > g0 ? (uint32_t)min(e1 - base, (uint64_t)32) : 0u);
     }
-    uint32_t pos[NP];
-    coop_find32<NP>(B, pool, line, blh, x, f, pos);
-#pragma unroll
-    for (int k = 0; k < NP; k++) q[k] = (bon[k] && pos[k] < 32) ? 32ull * line[k] + pos[k] : kNoPos;
+    const uint32_t pos = coop_find32<POS, false>(in, (uint32_t)(base >> 5), vm, false, x);
+    return (vm && pos < 32) ? base + pos : kNoPos;
 }
 
 template <int NT, int KS, int MAXSEG, int CAPB, bool BSR, bool COUNT_ONLY, int SMODE, bool DIRECT = false>
@@ -577,48 +561,81 @@ __global__ __launch_bounds__(NT, 4) void search_tile_kernel(PairBatch in, TilePl
         }
         __syncthreads();
 
-        // ---- 2. narrow the larger sets: one wave per segment ----------------------------------------
-        // A larger set in an indexed B pool longer than kNoNarrow elements is not narrowed: its
-        // window could be staged only if the probes clustered, and the two 64-way searches would
-        // cost more HBM lines than the probes themselves; every probe finds its line through the
-        // index instead.
-        for (uint32_t s = wave; s < nseg; s += NW) {
-            const uint32_t n = sm.seg_wa[s];
-            const uint32_t nl = sm.seg_hi[s];
-            uint32_t lo = 0, hi = 0;
-            if (n && in.b_idx && !((sm.seg_flags[s] >> 2) & 1u) && nl > kNoNarrow) {
-                hi = nl;
-            } else if (n) {
+        // ---- 2. narrow the larger sets of the pairs that other tiles share ----------------------------
+        // At most the first and the last segment are parts of a pair; their probes reach only a
+        // part of the larger set, whose bounds four waves find, one 64-way search each.  A pair that
+        // lies whole in the tile searches its whole larger set: narrowing one would cost two
+        // searches of dependent reads, one pair after another (a tile of 130 small pairs waited for
+        // 33 of them).  A larger set longer than kNoNarrow in an indexed pool whose top level is
+        // staged is not narrowed either: every probe finds its line through the index.
+        static_assert(NW == 4, "one wave per bound");
+        auto through_index = [&](uint32_t swapped, uint32_t nl) {
+            return top_ok && in.b_idx && !swapped && nl > kNoNarrow;
+        };
+        auto partial = [&](uint32_t s) {
+            const uint32_t f = sm.seg_flags[s];
+            return sm.seg_wa[s] && (f & 3u) != 3u && !through_index((f >> 2) & 1u, sm.seg_hi[s]);
+        };
+        if (nseg) {
+            const uint32_t s = wave < 2 ? 0u : nseg - 1;
+            if ((wave < 2 || s != 0) && partial(s)) {
                 const bool large_is_a = (sm.seg_flags[s] >> 2) & 1u;
                 const uint32_t *__restrict__ L = (large_is_a ? in.A : in.B) + sm.seg_lbase[s];
-                const uint32_t vf = sm.pkey[sm.seg_la[s]], vl = sm.pkey[sm.seg_la[s] + n - 1];
-                const uint32_t f = in.sflip;
-                lo = (uint32_t)group_partition_point<kWave>(0, nl, lane, 0, [&](uint64_t x) { return (L[x] ^ f) < vf; });
-                hi = (uint32_t)group_partition_point<kWave>(lo, nl, lane, 0, [&](uint64_t x) { return (L[x] ^ f) <= vl; });
-            }
-            if (lane == 0) {
-                sm.seg_lo[s] = lo;
-                sm.seg_hi[s] = hi;
+                const uint32_t nl = sm.seg_hi[s], f = in.sflip;
+                const uint32_t v = sm.pkey[sm.seg_la[s] + ((wave & 1u) ? sm.seg_wa[s] - 1 : 0u)];
+                const bool up = (wave & 1u) != 0;
+                const uint32_t r = (uint32_t)group_partition_point<kWave>(0, nl, lane, 0, [&](uint64_t x) {
+                    const uint32_t y = L[x] ^ f;
+                    return up ? y <= v : y < v;
+                });
+                if (lane == 0) sm.narrow[wave] = r;
             }
         }
         __syncthreads();
 
-        // ---- 3. stage the narrowed larger windows while they fit --------------------------------------
+        // ---- 3. stage or sample the larger windows while they fit -------------------------------------
+        // A window of at most kStage elements per probe is staged whole.  Of a longer one LDS gets
+        // the first element of every m-th 128-byte line: at most kSample samples per probe, each
+        // line's read when it is the one that can hold a probe (4a).  So a probe costs at most kSample
+        // lines of samples (fewer through the index) and one line of the set, in two round trips,
+        // where a gallop or binary search from the window's start reads a line per level.  The limits
+        // are what LDS holds beside four workgroups per CU.  (3,000 pairs of larger sets of 2^12 to
+        // 2^16 elements and ratios up to 4,096: the whole batch 279 us with narrowed windows searched
+        // in global memory, 239 us sampled, 208 us with 4a.)
+        uint32_t nst = 0;   // segments whose windows fit
+        uint32_t ltot = 0;  // chunks of staged and sampled windows (0: every probe goes through the index)
+        constexpr uint32_t kStage = CAPB / U - 1, kSample = CAPB / U > 5 ? 4 : CAPB / U - 1, kMinSample = 24;
         {
-            uint32_t cl = 0;
+            uint32_t cl = 0, m = 0, ns = 0, lo = 0, hi = 0;
             uint64_t gl = 0;
             uint32_t src = 0;
+            bool idx = false;
             if (tid < nseg) {
-                const uint32_t n = sm.seg_hi[tid] - sm.seg_lo[tid];
-                gl = sm.seg_lbase[tid] + sm.seg_lo[tid];
-                src = ((sm.seg_flags[tid] >> 2) & 1u) ? 0u : 1u;  // pool of the larger side
-                cl = n ? ((uint32_t)(gl & 3) + n + 3) / 4 : 0u;
+                const uint32_t k = sm.seg_wa[tid], f = sm.seg_flags[tid];
+                idx = through_index((f >> 2) & 1u, sm.seg_hi[tid]);
+                hi = k ? sm.seg_hi[tid] : 0u;
+                if (partial(tid) && (tid == 0 || tid == nseg - 1)) {
+                    lo = sm.narrow[tid == 0 ? 0 : 2];
+                    hi = sm.narrow[tid == 0 ? 1 : 3];
+                }
+                const uint32_t n = hi - lo;
+                gl = sm.seg_lbase[tid] + lo;
+                src = ((f >> 2) & 1u) ? 0u : 1u;  // pool of the larger side
+                if (idx || n == 0) {
+                    cl = 0;
+                } else if (n <= kStage * k) {
+                    cl = ((uint32_t)(gl & 3) + n + 3) / 4;
+                } else {
+                    const uint32_t heads = (uint32_t)(((gl + n - 1) >> 5) - (gl >> 5));  // lines after the first
+                    const uint32_t most = max(kSample * k, kMinSample);
+                    m = max((heads + most - 1) / most, 1u);
+                    ns = heads / m;
+                    cl = max((ns + 3) / 4, 1u);
+                }
             }
-            uint32_t ltot = 0;
             const uint32_t lpfx = block_exclusive_scan<NT>(cl, sm.scan_scratch, &ltot);
             const bool fits = lpfx + cl <= (uint32_t)(CAPB / 4);
-            // staged segments form a prefix; their count is the number of fitting threads
-            uint32_t nst = 0;
+            // the segments that fit form a prefix; their count is the number of fitting threads
             {
                 const uint64_t bal = ballot(tid < nseg && fits);
                 if (lane == 0) sm.wave_el[wave] = (uint32_t)__popcll(bal);
@@ -626,11 +643,15 @@ __global__ __launch_bounds__(NT, 4) void search_tile_kernel(PairBatch in, TilePl
             __syncthreads();
             for (int k = 0; k < NW; k++) nst += sm.wave_el[k];
             if (tid < nseg) {
+                sm.seg_lo[tid] = lo;
+                sm.seg_hi[tid] = hi;
+                sm.seg_m[tid] = m;
+                sm.seg_flags[tid] |= ns << 8;
                 if (fits) {
                     sm.win_c[tid] = lpfx;
-                    sm.win_g[tid] = gl & ~3ull;
+                    sm.win_g[tid] = m ? gl : gl & ~3ull;
                     sm.win_src[tid] = src;
-                    sm.seg_lb[tid] = 4u * lpfx + (uint32_t)(gl & 3);
+                    sm.seg_lb[tid] = idx ? kNotStaged : 4u * lpfx + (m ? 0u : (uint32_t)(gl & 3));
                 } else {
                     sm.seg_lb[tid] = kNotStaged;
                 }
@@ -639,12 +660,11 @@ __global__ __launch_bounds__(NT, 4) void search_tile_kernel(PairBatch in, TilePl
             if (tid == 0 && nst == 0) sm.win_c[0] = 0;
             __syncthreads();
             if (nst) {
-                constexpr int QL = (Smem::LKEYS + 4 * NT - 1) / (4 * NT);
-                stage_windows<NT, QL>(in.A, in.a_pool, in.B, in.b_pool, sm.win_c, sm.win_g, sm.win_src, nst, sm.lkey,
-                                      in.sflip);
+                constexpr int QL = (CAPB + 4 * NT - 1) / (4 * NT);
+                stage_or_sample<NT, QL>(in, sm.win_c, sm.win_g, sm.win_src, sm.seg_m, sm.seg_flags, nst, sm.lkey);
                 if constexpr (BSR)
                     stage_windows<NT, QL>(in.As, in.a_pool, in.Bs, in.b_pool, sm.win_c, sm.win_g, sm.win_src, nst,
-                                          sm.lst, 0u);
+                                          sm.lst, 0u, sm.seg_m);
             }
             __syncthreads();
         }
@@ -688,124 +708,208 @@ __global__ __launch_bounds__(NT, 4) void search_tile_kernel(PairBatch in, TilePl
             }
             s0 = lo;
         }
-        // 4a. probes answered through the indexed B pool with its top level staged: looked up
-        // first, the whole wave together (coop_index_probe_top), the k-th probe of every lane at
-        // once; qrel[k] is the found position relative to the larger set, or ~0.  A probe's range
-        // starts at its narrowed window rather than at the previous hit: a set holds x once, so the
-        // position found is the same.
-        uint32_t qrel[KS];
-#pragma unroll
-        for (int k = 0; k < KS; k++) qrel[k] = ~0u;
-        if (top_ok && in.b_idx) {
-            // one probe per lane at a time (two at once, NP = 2, measured no faster at two probes
-            // per lane and slower at four, where the registers of the second cost occupancy)
-            constexpr int NP = 1;
-            uint32_t s = s0;
-#pragma unroll
-            for (int k0 = 0; k0 < KS; k0 += NP) {
-                bool on[NP];
-                uint32_t x[NP];
-                uint64_t g[NP], g0[NP], g1[NP], q[NP];
-                bool any = false;
-#pragma unroll
-                for (int j = 0; j < NP; j++) {
-                    const uint32_t u = ub + (uint32_t)(k0 + j);
-                    on[j] = k0 + j < KS && u < ulen;
-                    x[j] = 0;
-                    g[j] = g0[j] = g1[j] = 0;
-                    if (on[j]) {
-                        while (u >= sm.seg_u[s + 1]) s++;
-                        const uint32_t e = u - sm.seg_u[s];
-                        on[j] = e < sm.seg_wa[s] && sm.seg_lb[s] == kNotStaged && !((sm.seg_flags[s] >> 2) & 1u);
-                        if (on[j]) {
-                            x[j] = sm.pkey[sm.seg_la[s] + e];
-                            g[j] = sm.seg_lbase[s];
-                            g0[j] = g[j] + sm.seg_lo[s];
-                            g1[j] = g[j] + sm.seg_hi[s];
-                        }
-                    }
-                    any = any || on[j];
-                }
-                if (ballot(any) != 0) {  // wave-uniform
-                    coop_index_probe_top<NP>(on, in.B, in.b_pool, in.b_idx, in.b_mid, sm.top, tj0, g0, g1, x, in.sflip,
-                                             q);
-#pragma unroll
-                    for (int j = 0; j < NP; j++)
-                        if (k0 + j < KS && q[j] != kNoPos) qrel[k0 + j] = (uint32_t)(q[j] - g[j]);
-                }
-            }
-        }
-        if (ub < ulen) {
-            uint32_t s = s0;
-            uint32_t cur = sm.seg_lo[s];  // pair-relative position in the larger set
+        // fmask: the lane's probes found (bit k); BSR also keeps their states in the larger set.  A set
+        // holds x at most once, so where a search starts does not change what it finds.  (Four probes
+        // per lane: the loops of 4a and 4b are not unrolled, so that a lookup's registers are held once.)
+        constexpr int UK = (BSR || KS <= 2) ? KS : 1;
+        uint32_t fmask = 0;
+        uint32_t lstate[BSR ? KS : 1];
+        // 4a. probes of windows staged whole: binary lifting in LDS with the wave's common steps, the KS
+        // searches in lockstep, so that their reads overlap (two probes, windows of up to 3,000
+        // elements: 2,900 cycles where galloping through them in turn takes 6,500)
+        if (ltot) {
+            uint32_t at[KS], end[KS], xv[KS], nmax = 0, s = s0;
 #pragma unroll
             for (int k = 0; k < KS; k++) {
                 const uint32_t u = ub + (uint32_t)k;
-                if (u >= ulen) break;
-                if (u >= sm.seg_u[s + 1]) {
-                    s++;
-                    cur = sm.seg_lo[s];
-                }
-                const uint32_t e = u - sm.seg_u[s];
-                if (e >= sm.seg_wa[s]) continue;  // padding unit
-                const uint32_t x = sm.pkey[sm.seg_la[s] + e];
-                const uint32_t lo_s = sm.seg_lo[s], hi_s = sm.seg_hi[s], lb = sm.seg_lb[s];
-                const bool large_is_a = (sm.seg_flags[s] >> 2) & 1u;
-                uint32_t pos;
-                bool found;
-                uint32_t lstate = 0;
-                if (lb != kNotStaged) {
-                    auto arr = [&](uint32_t i) { return sm.lkey[lb + (i - lo_s)]; };
-                    if constexpr (SMODE == SM_BLOCK) pos = lower_bound_block<kBlockLds>(arr, cur, hi_s, x);
-                    else pos = lower_bound_from<SMODE == SM_GALLOP>(arr, cur, hi_s, x);
-                    found = pos < hi_s && arr(pos) == x;
-                    if constexpr (BSR)
-                        if (found) lstate = sm.lst[lb + (pos - lo_s)];
-                } else if (in.b_idx && !large_is_a) {
-                    // resident B pool with an index of every 32nd element: binary search the index,
-                    // then compare one 128-byte line of B (with the top level staged: looked up in 4a)
-                    const uint64_t g = sm.seg_lbase[s];
-                    const uint64_t q = top_ok ? (qrel[k] != ~0u ? g + qrel[k] : kNoPos)
-                                              : index_probe(in.B, in.b_pool, in.b_idx, in.b_mid, g + cur, g + hi_s, x,
-                                                            in.sflip);
-                    found = q != kNoPos;
-                    pos = found ? (uint32_t)(q - g) : cur;
-                    if constexpr (BSR)
-                        if (found) lstate = in.Bs[q];
-                } else {
-                    if constexpr (SMODE == SM_BLOCK) {
-                        pos = lower_bound_block_pool(large_is_a ? in.A : in.B, large_is_a ? in.a_pool : in.b_pool,
-                                                     sm.seg_lbase[s], cur, hi_s, x, in.sflip, found);
-                    } else {
-                        const uint32_t *__restrict__ L = (large_is_a ? in.A : in.B) + sm.seg_lbase[s];
-                        const uint32_t f = in.sflip;
-                        auto arr = [&](uint32_t i) { return L[i] ^ f; };
-                        pos = lower_bound_from<SMODE == SM_GALLOP>(arr, cur, hi_s, x);
-                        found = pos < hi_s && arr(pos) == x;
+                at[k] = end[k] = 1;
+                xv[k] = 0;
+                if (u < ulen) {
+                    while (u >= sm.seg_u[s + 1]) s++;
+                    const uint32_t e = u - sm.seg_u[s], lb = sm.seg_lb[s];
+                    if (e < sm.seg_wa[s] && lb != kNotStaged && sm.seg_m[s] == 0) {
+                        const uint32_t n = sm.seg_hi[s] - sm.seg_lo[s];
+                        xv[k] = sm.pkey[sm.seg_la[s] + e];
+                        at[k] = lb;
+                        end[k] = lb + n;
+                        nmax = max(nmax, n);
                     }
-                    if constexpr (BSR)
-                        if (found) lstate = (large_is_a ? in.As : in.Bs)[sm.seg_lbase[s] + pos];
                 }
-                cur = pos;
-                if constexpr (!BSR) {
-                    // further sets in order; the first one that lacks x ends the lookup
-                    for (uint32_t j = 0; found && j < nx; j++) {
+            }
+            const uint32_t L = wave_max_u32(32u - (uint32_t)__clz(nmax));
+            for (int bit = (int)L - 1; bit >= 0; bit--) {
+#pragma unroll
+                for (int k = 0; k < KS; k++) {
+                    const uint32_t y = min(at[k] + (1u << bit), end[k]);
+                    // (at its window's end, or without one, a probe stays: y == at)
+                    if (sm.lkey[y - 1] < xv[k]) at[k] = y;
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < KS; k++) {
+                const bool found = at[k] < end[k] && sm.lkey[at[k]] == xv[k];
+                fmask |= found ? 1u << k : 0u;
+                if constexpr (BSR) lstate[k] = found ? sm.lst[at[k]] : 0u;
+            }
+        }
+        // 4b. probes of sampled windows, the whole wave together, the k-th probe of every lane at once:
+        // the samples at most x give the m lines that can hold it, a search over those lines' first
+        // elements (m > 1) the one line, which a group of lanes reads.
+        if (ltot) {
+            uint32_t s = s0;
+#pragma unroll UK
+            for (int k = 0; k < KS; k++) {
+                const uint32_t u = ub + (uint32_t)k;
+                uint32_t x = 0, line = 0, vm = 0;
+                bool in_a = false;
+                if (u < ulen) {
+                    while (u >= sm.seg_u[s + 1]) s++;
+                    const uint32_t e = u - sm.seg_u[s];
+                    const uint32_t m = sm.seg_m[s], lb = sm.seg_lb[s];
+                    if (m && lb != kNotStaged && e < sm.seg_wa[s]) {
+                        x = sm.pkey[sm.seg_la[s] + e];
+                        const uint32_t f = sm.seg_flags[s];
+                        const bool large_is_a = (f >> 2) & 1u;
+                        const uint64_t base = sm.seg_lbase[s];
+                        const uint64_t g0 = base + sm.seg_lo[s], g1 = base + sm.seg_hi[s];
+                        uint32_t lo = 0, hi = f >> 8;  // samples at most x
+                        while (lo < hi) {
+                            const uint32_t mid = (lo + hi) >> 1;
+                            if (sm.lkey[lb + mid] <= x) lo = mid + 1; else hi = mid;
+                        }
+                        line = (uint32_t)(g0 >> 5) + lo * m;
+                        if (m > 1) {
+                            const uint32_t end = (uint32_t)((g1 - 1) >> 5) + 1;
+                            uint32_t n = min(m, end - line);  // the last of n lines whose first element is at most x
+                            while (n > 1) {
+                                const uint32_t h = n >> 1, q = line + h;
+                                const uint32_t y = (in.b_idx && !large_is_a)
+                                                       ? in.b_idx[q]
+                                                       : (large_is_a ? in.A : in.B)[32ull * q] ^ in.sflip;
+                                if (y <= x) {
+                                    line = q;
+                                    n -= h;
+                                } else {
+                                    n = h;
+                                }
+                            }
+                        }
+                        const uint64_t l0 = 32ull * line;
+                        const uint32_t from = g0 > l0 ? (uint32_t)(g0 - l0) : 0u;
+                        vm = line_mask(from, (uint32_t)min(g1 - l0, (uint64_t)32));
+                        in_a = large_is_a;
+                    }
+                }
+                if (ballot(vm != 0) != 0) {  // wave-uniform
+                    const uint32_t pos = coop_find32<BSR, true>(in, line, vm, in_a, x);
+                    if (vm && pos < 32) {
+                        fmask |= 1u << k;
+                        if constexpr (BSR) lstate[k] = (in_a ? in.As : in.Bs)[32ull * line + pos];
+                    }
+                }
+            }
+        }
+        // probes answered through the indexed B pool with its top level staged, likewise
+        if (top_ok && in.b_idx) {
+            // one probe per lane at a time (two at once measured no faster at two probes per lane and
+            // slower at four, where the registers of the second cost occupancy)
+            uint32_t s = s0;
+#pragma unroll UK
+            for (int k = 0; k < KS; k++) {
+                const uint32_t u = ub + (uint32_t)k;
+                bool on = u < ulen;
+                uint32_t x = 0;
+                uint64_t g0 = 0, g1 = 0;
+                if (on) {
+                    while (u >= sm.seg_u[s + 1]) s++;
+                    const uint32_t e = u - sm.seg_u[s];
+                    on = e < sm.seg_wa[s] && sm.seg_lb[s] == kNotStaged && !((sm.seg_flags[s] >> 2) & 1u);
+                    if (on) {
+                        x = sm.pkey[sm.seg_la[s] + e];
+                        g0 = sm.seg_lbase[s] + sm.seg_lo[s];
+                        g1 = sm.seg_lbase[s] + sm.seg_hi[s];
+                    }
+                }
+                if (ballot(on) != 0) {  // wave-uniform
+                    const uint64_t q = coop_index_probe_top<BSR>(in, on, sm.top, tj0, g0, g1, x);
+                    if (q != kNoPos) {
+                        fmask |= 1u << k;
+                        if constexpr (BSR) lstate[k] = in.Bs[q];
+                    }
+                }
+            }
+        }
+        // 4c. probes of windows that found no room in LDS, each by its lane
+        if (nst < nseg && ub < ulen) {
+            uint32_t s = s0;
+#pragma unroll UK
+            for (int k = 0; k < KS; k++) {
+                const uint32_t u = ub + (uint32_t)k;
+                if (u >= ulen) break;
+                while (u >= sm.seg_u[s + 1]) s++;
+                const uint32_t e = u - sm.seg_u[s];
+                const bool large_is_a = (sm.seg_flags[s] >> 2) & 1u, idx = in.b_idx && !large_is_a;
+                if (e >= sm.seg_wa[s] || sm.seg_lb[s] != kNotStaged || (idx && top_ok)) continue;
+                const uint32_t x = sm.pkey[sm.seg_la[s] + e], lo = sm.seg_lo[s], hi = sm.seg_hi[s];
+                const uint64_t g = sm.seg_lbase[s];
+                bool found;
+                uint64_t q = 0;
+                if (idx) {
+                    // the index, then one 128-byte line
+                    q = index_probe(in.B, in.b_pool, in.b_idx, in.b_mid, g + lo, g + hi, x, in.sflip);
+                    found = q != kNoPos;
+                } else if constexpr (SMODE == SM_BLOCK) {
+                    q = g + lower_bound_block_pool(large_is_a ? in.A : in.B, large_is_a ? in.a_pool : in.b_pool, g, lo,
+                                                   hi, x, in.sflip, found);
+                } else {
+                    const uint32_t *__restrict__ L = (large_is_a ? in.A : in.B) + g;
+                    const uint32_t f = in.sflip;
+                    auto arr = [&](uint32_t i) { return L[i] ^ f; };
+                    const uint32_t pos = lower_bound_from<SMODE == SM_GALLOP>(arr, lo, hi, x);
+                    found = pos < hi && arr(pos) == x;
+                    q = g + pos;
+                }
+                if (found) {
+                    fmask |= 1u << k;
+                    if constexpr (BSR) lstate[k] = (large_is_a ? in.As : in.Bs)[q];
+                }
+            }
+        }
+        hmask = fmask;
+        if constexpr (BSR) {
+            // a base match is a result when the state AND is non-zero
+            uint32_t s = s0;
+#pragma unroll
+            for (int k = 0; k < KS; k++) {
+                svals[k] = 0;
+                if ((fmask >> k) & 1u) {
+                    const uint32_t u = ub + (uint32_t)k;
+                    while (u >= sm.seg_u[s + 1]) s++;
+                    svals[k] = sm.pst[sm.seg_la[s] + (u - sm.seg_u[s])] & lstate[k];
+                    nelems += __popc(svals[k]);
+                    if (!svals[k]) hmask &= ~(1u << k);
+                }
+            }
+        }
+        if constexpr (!BSR) {
+            // further sets of a single pair, in order; the first one that lacks x ends the lookup
+            if (nx) {
+                for (uint32_t m = fmask; m; m &= m - 1) {
+                    const uint32_t k = __builtin_ctz(m);
+                    const uint32_t x = sm.pkey[sm.seg_la[0] + (ub + k - sm.seg_u[0])], f = in.sflip;
+                    bool found = true;
+#pragma unroll
+                    for (uint32_t j = 0; j < (uint32_t)kMaxExtraSets; j++) {
+                        if (!found || j >= nx) continue;
                         const uint32_t *__restrict__ X = in.xsets[j];
-                        const uint32_t f = in.sflip;
                         auto xarr = [&](uint32_t i) { return X[i] ^ f; };
                         const uint32_t xh = sm.xhi[j];
                         const uint32_t xp = lower_bound_from<SMODE != SM_BINARY>(xarr, xcur[j], xh, x);
                         xcur[j] = xp;
                         found = xp < xh && xarr(xp) == x;
                     }
+                    if (!found) hmask &= ~(1u << k);
                 }
-                if constexpr (BSR) {
-                    const uint32_t stv = found ? (sm.pst[sm.seg_la[s] + e] & lstate) : 0u;
-                    found = stv != 0;
-                    svals[k] = stv;
-                    nelems += __popc(stv);
-                }
-                hmask |= found ? (1u << k) : 0u;
             }
         }
         if constexpr (!BSR) {

@@ -86,7 +86,10 @@ static_assert(pad_for(kNTM * 12, kMaxSeg) >= 12 && pad_for(kNTM * 20, kMaxSeg) >
                   pad_for(kNTM * kBsrK, kMaxSeg) >= kBsrK && pad_for(kNT * 1, kMaxSeg) >= 1 &&
                   pad_for(kNTM * 12, kMaxSegGather) >= 12 && pad_for(kNTM * 24, kMaxSegGather) >= 24,
               "a lane crosses at most one pair boundary");
-constexpr int kCapB = 3072;  // search policy: larger windows staged up to this many words
+// search policy: words of staged or sampled larger windows per tile (BSR tiles hold states too; both
+// leave the workgroups per CU that the registers allow: four, BSR three)
+constexpr int kCapB = 3584;
+constexpr int kCapBBsr = 2560;
 
 constexpr uint32_t kOneScanGroups = 8;      // pair-unit scans of up to this many groups run as one workgroup
 constexpr uint32_t kOneScanParts = 32;      // ... on at most this many workgroups, each with all the sizes
@@ -536,7 +539,7 @@ void launch_search_t(setops_hip_batch *h, const TileOut &out, hipStream_t stream
         }
     }
     for (uint64_t t0 = 0; t0 < h->plan.ntiles; t0 += kMaxGrid)
-        hipLaunchKernelGGL((search_tile_kernel<kNT, KS, kMaxSeg, kCapB, BSR, CO, SMODE>),
+        hipLaunchKernelGGL((search_tile_kernel<kNT, KS, kMaxSeg, BSR ? kCapBBsr : kCapB, BSR, CO, SMODE>),
                            dim3((uint32_t)std::min<uint64_t>(kMaxGrid, h->plan.ntiles - t0)), dim3(kNT), 0, stream,
                            h->in, h->plan, out, (uint32_t)t0);
 }

@@ -895,11 +895,13 @@ __device__ __forceinline__ void stage_run_lds(const uint32_t *__restrict__ src, 
 // the windows' chunk counts (cpfx[nwin] = total).  Each thread takes chunks c, c + NT, ... (at most
 // QMAX of them), finds each chunk's window by binary search over cpfx, and issues all its loads
 // before storing.  Every staged word is XORed with `flip` (PairBatch::sflip for keys, 0 for states).
+// With `skip`, windows of a non-zero skip[w] are left out.
 template <int NT, int QMAX>
 __device__ __forceinline__ void stage_windows(const uint32_t *__restrict__ srcA, uint64_t poolA,
                                               const uint32_t *__restrict__ srcB, uint64_t poolB,
                                               const uint32_t *cpfx, const uint64_t *gbase, const uint32_t *wsrc,
-                                              uint32_t nwin, uint32_t *dst, uint32_t flip)
+                                              uint32_t nwin, uint32_t *dst, uint32_t flip,
+                                              const uint32_t *skip = nullptr)
 {
     const uint32_t total = cpfx[nwin];
     uint4 v[QMAX];
@@ -913,7 +915,8 @@ __device__ __forceinline__ void stage_windows(const uint32_t *__restrict__ srcA,
                 if (cpfx[mid] <= c) lo = mid; else hi = mid;
             }
             const bool fromB = wsrc[lo] != 0;
-            v[k] = load_chunk(fromB ? srcB : srcA, fromB ? poolB : poolA, gbase[lo] + 4ull * (c - cpfx[lo]));
+            if (skip && skip[lo]) v[k] = make_uint4(0u, 0u, 0u, 0u);
+            else v[k] = load_chunk(fromB ? srcB : srcA, fromB ? poolB : poolA, gbase[lo] + 4ull * (c - cpfx[lo]));
         }
     }
 #pragma unroll
@@ -927,6 +930,55 @@ __device__ __forceinline__ void stage_windows(const uint32_t *__restrict__ srcA,
             x.w ^= flip;
             *reinterpret_cast<uint4 *>(dst + 4 * c) = x;
         }
+    }
+}
+
+// stage_windows for the larger windows of a search tile (keys): window w is staged whole where
+// m[w] == 0; else it is the samples j < flags[w] >> 8, the first elements of the pool's 32-element
+// lines (g0_w >> 5) + (j + 1) m[w] (from the index where B has one), in the compare space.
+template <int NT, int QMAX>
+__device__ __forceinline__ void stage_or_sample(const PairBatch &in, const uint32_t *cpfx, const uint64_t *gbase,
+                                                const uint32_t *wsrc, const uint32_t *m, const uint32_t *flags,
+                                                uint32_t nwin, uint32_t *dst)
+{
+    const uint32_t total = cpfx[nwin];
+    uint4 v[QMAX];
+#pragma unroll
+    for (int k = 0; k < QMAX; k++) {
+        const uint32_t c = threadIdx.x + (uint32_t)k * NT;
+        v[k] = make_uint4(0u, 0u, 0u, 0u);
+        if (c < total) {
+            uint32_t lo = 0, hi = nwin;  // largest w with cpfx[w] <= c
+            while (hi - lo > 1) {
+                const uint32_t mid = (lo + hi) >> 1;
+                if (cpfx[mid] <= c) lo = mid; else hi = mid;
+            }
+            const bool fromB = wsrc[lo] != 0;
+            const uint32_t *__restrict__ src = fromB ? in.B : in.A;
+            const uint64_t g = gbase[lo];
+            const uint32_t mw = m[lo], j0 = 4u * (c - cpfx[lo]);
+            if (mw == 0) {
+                v[k] = load_chunk(src, fromB ? in.b_pool : in.a_pool, g + j0);
+                v[k].x ^= in.sflip;
+                v[k].y ^= in.sflip;
+                v[k].z ^= in.sflip;
+                v[k].w ^= in.sflip;
+            } else {
+                const bool idx = fromB && in.b_idx;
+                const uint32_t *__restrict__ p = idx ? in.b_idx : src;
+                const uint32_t ns = flags[lo] >> 8, sh = idx ? 0u : 5u, f = idx ? 0u : in.sflip;
+                const uint64_t l0 = (g >> 5) + (uint64_t)(j0 + 1) * mw;
+                if (j0 + 0 < ns) v[k].x = p[l0 << sh] ^ f;
+                if (j0 + 1 < ns) v[k].y = p[(l0 + mw) << sh] ^ f;
+                if (j0 + 2 < ns) v[k].z = p[(l0 + 2ull * mw) << sh] ^ f;
+                if (j0 + 3 < ns) v[k].w = p[(l0 + 3ull * mw) << sh] ^ f;
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < QMAX; k++) {
+        const uint32_t c = threadIdx.x + (uint32_t)k * NT;
+        if (c < total) *reinterpret_cast<uint4 *>(dst + 4 * c) = v[k];
     }
 }
 
