@@ -559,7 +559,7 @@ __global__ __launch_bounds__(NT) void merge_tile_kernel(PairBatch in, TilePlan p
         if (bad) nseg = 0;
         if (t == 0 && tid == 0 && out.error && !direct && plan.uoff[in.P] != plan.utotal) atomicOr(out.error, 4u);
         SegWin w{};
-        uint32_t staged_words = 0;  // CSR: words loaded straight into LDS (flipped in place for int32 sets)
+        uint32_t staged_words = 0;  // words loaded straight into LDS (flipped in place for int32 sets)
         uint32_t bstart = 0;        // key index where the staged B words start
 
         // ---- 2. stage the windows --------------------------------------------------------------
@@ -621,14 +621,8 @@ __global__ __launch_bounds__(NT) void merge_tile_kernel(PairBatch in, TilePlan p
             staged_words = 4u * (totA + totB);
             bstart = 4u * totA;
             __syncthreads();
-            constexpr int QWIN = (Smem::KEYS + 4 * NT - 1) / (4 * NT);
-            if (!bad) {
-                stage_windows<NT, QWIN>(in.A, in.a_pool, in.B, in.b_pool, sm.win_c, sm.win_g, sm.win_src, 2 * nseg,
-                                        sm.key, in.sflip);
-                if constexpr (BSR)
-                    stage_windows<NT, QWIN>(in.As, in.a_pool, in.Bs, in.b_pool, sm.win_c, sm.win_g, sm.win_src,
-                                            2 * nseg, sm.st, 0u);
-            }
+            if (!bad)
+                stage_windows_lds<NT, BSR>(in, sm.win_c, sm.win_g, sm.win_src, 2 * nseg, sm.key, sm.st);
         }
         if (bad) {
             nseg = 0;
@@ -644,9 +638,9 @@ __global__ __launch_bounds__(NT) void merge_tile_kernel(PairBatch in, TilePlan p
             sm.seg_nb[tid] = wb + (w.j1 < w.nb ? 1u : 0u);
         }
         if (tid == 0) sm.seg_u[nseg] = ulen;
-        if constexpr (!GATHER) __builtin_amdgcn_s_waitcnt(0);  // the direct-to-LDS loads have landed
+        __builtin_amdgcn_s_waitcnt(0);  // the direct-to-LDS loads have landed
         __syncthreads();
-        if constexpr (!GATHER && !BSR) {
+        if constexpr (!BSR) {
             // int32 sets: flip bit 31 of the staged words, so unsigned compares give signed order
             if (in.sflip) {
                 for (uint32_t i = tid; i < staged_words; i += NT) sm.key[i] ^= in.sflip;

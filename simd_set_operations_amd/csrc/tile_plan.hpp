@@ -933,6 +933,52 @@ __device__ __forceinline__ void stage_windows(const uint32_t *__restrict__ srcA,
     }
 }
 
+// stage_windows with direct global->LDS loads, a window at a time per wave (windows w, w + NT / 64, ...;
+// the wave's lanes hold their descriptions): no search for a chunk's window, no registers between
+// the load and LDS.  With states (ST) each window's are staged beside it, from srcAs / srcBs to dst_s.
+// The caller waits (s_waitcnt) and synchronizes before reading dst.
+template <int NT, bool ST>
+__device__ __forceinline__ void stage_windows_lds(const PairBatch &in, const uint32_t *cpfx, const uint64_t *gbase,
+                                                  const uint32_t *wsrc, uint32_t nwin, uint32_t *dst, uint32_t *dst_s)
+{
+    constexpr uint32_t NW = NT / kWave;
+    const uint32_t lane = lane_id();
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    const uint32_t w = wave + NW * lane;
+    uint32_t c = 0, n = 0, full = 0, b = 0;
+    uint64_t g = 0;
+    if (w < nwin) {
+        c = cpfx[w];
+        n = cpfx[w + 1] - c;
+        g = gbase[w];
+        b = wsrc[w];
+        // chunks that lie in the pool (the one that reaches past it, at most the last, goes word by word)
+        const uint64_t pool = b ? in.b_pool : in.a_pool;
+        const uint64_t fp = pool > g ? (pool - g) / 4 : 0;
+        full = (uint32_t)min((uint64_t)n, fp);
+    }
+    const uint32_t cnt = nwin > wave ? (nwin - wave + NW - 1) / NW : 0u;
+    for (uint32_t j = 0; j < cnt; j++) {
+        auto rl = [&](uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)j); };
+        const uint32_t jc = rl(c), jn = rl(n), jf = rl(full), jb = rl(b);
+        const uint64_t jg = (uint64_t)rl((uint32_t)(g >> 32)) << 32 | rl((uint32_t)g);
+        const uint4 *p = reinterpret_cast<const uint4 *>((jb ? in.B : in.A) + jg);
+        for (uint32_t r = 0; r < jf; r += kWave)
+            if (r + lane < jf) {
+                __builtin_amdgcn_global_load_lds(p + r + lane, dst + 4 * (jc + r), 16, 0, 0);
+                if constexpr (ST)
+                    __builtin_amdgcn_global_load_lds(reinterpret_cast<const uint4 *>((jb ? in.Bs : in.As) + jg) + r + lane,
+                                                     dst_s + 4 * (jc + r), 16, 0, 0);
+            }
+        if (jf < jn && lane < 4) {
+            const uint64_t e = jg + 4ull * jf + lane;
+            const bool ok = e < (jb ? in.b_pool : in.a_pool);
+            dst[4 * (jc + jf) + lane] = ok ? (jb ? in.B : in.A)[e] : 0u;
+            if constexpr (ST) dst_s[4 * (jc + jf) + lane] = ok ? (jb ? in.Bs : in.As)[e] : 0u;
+        }
+    }
+}
+
 // stage_windows for the larger windows of a search tile (keys): window w is staged whole where
 // m[w] == 0; else it is the samples j < flags[w] >> 8, the first elements of the pool's 32-element
 // lines (g0_w >> 5) + (j + 1) m[w] (from the index where B has one), in the compare space.
