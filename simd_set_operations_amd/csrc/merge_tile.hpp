@@ -164,7 +164,7 @@ __device__ __forceinline__ uint32_t block_intersect(const uint32_t *key, const u
 
 // Steps 3-6 of a tile whose windows and segment table are in LDS (seg_* arrays, key/st): the
 // lanes' merge (or block policy), the tile scan, staged outputs, tile and per-pair counts.
-template <int NT, int K, int MAXSEG, bool BSR, bool COUNT_ONLY, bool GATHER, int LP>
+template <int NT, int K, int MAXSEG, bool BSR, bool COUNT_ONLY, bool GATHER, int LP, bool DIRECT>
 __device__ __forceinline__ void merge_tile_compute(MergeSmem<NT, K, MAXSEG, BSR, GATHER, LP != LP_MERGE> &sm,
                                                    const TilePlan &plan, const TileOut &out, uint32_t t,
                                                    uint32_t nseg, uint32_t ulen, uint32_t p_first, uint32_t in_sflip,
@@ -478,9 +478,12 @@ __device__ __forceinline__ void merge_tile_compute(MergeSmem<NT, K, MAXSEG, BSR,
             }
             plan.tile_count[t] = tot;
             plan.tile_elems[t] = el;
-            if (plan.direct && out.totals) {  // one tile: its counts are the totals
-                out.totals[0] = tot;
-                out.totals[1] = el;
+            if (DIRECT && plan.one_tile) {  // its counts are the totals, its results the output
+                if (out.totals) {
+                    out.totals[0] = tot;
+                    out.totals[1] = el;
+                }
+                if (out.out_off) out.out_off[plan.single ? 1 : p_first + nseg] = tot;
             }
         }
         if (tid < nseg) {
@@ -504,12 +507,42 @@ __device__ __forceinline__ void merge_tile_compute(MergeSmem<NT, K, MAXSEG, BSR,
             const uint32_t f = sm.seg_flags[tid];
             const uint64_t p = (uint64_t)p_first + tid;
             if (f & 1u) plan.pair_local[p] = c0v;
-            if (out.counts) {
+            if (DIRECT && plan.one_tile && out.out_off) out.out_off[p] = c0v;  // every pair lies in the one tile
+            if (out.counts && (!DIRECT || plan.one_tile)) {  // else the placement writes them
                 if ((f & 3u) == 3u) out.counts[p] = c;
                 else if (c) atomicAdd(&out.counts[p], c);
             }
         }
     }
+}
+
+// Where unit v of a CSR batch or a single pair lies: its pair, the pair's split there (A and B index,
+// pair-relative and in the pools), and whether it is the pair's first unit.
+struct TileStart {
+    uint64_t ga, gb;
+    uint32_t pair, sa, sb, at_start;
+};
+
+// Found by a whole wave: v <= the unit total.
+__device__ __forceinline__ TileStart tile_start(const PairBatch &in, const TilePlan &plan, uint64_t v, uint32_t lane)
+{
+    uint64_t p = 0, a = 0, b = 0, na = plan.single_na, nb = plan.single_nb, u = 0;
+    if (!plan.single) {
+        p = group_partition_point<kWave>(1, in.P, lane, 0, [&](uint64_t x) { return csr_unit(in, plan.c0, x) <= v; }) - 1;
+        a = in.a_beg[p];
+        b = in.b_beg[p];
+        na = in.a_end[p] - a;
+        nb = in.b_end[p] - b;
+        u = csr_unit(in, plan.c0, p);
+    }
+    const uint64_t rel = v - u, d = rel < na + nb ? rel : na + nb;
+    const uint32_t *__restrict__ A = in.A + a;
+    const uint32_t *__restrict__ B = in.B + b;
+    const uint32_t f = in.sflip;
+    const uint64_t i = group_partition_point<kWave>(d > nb ? d - nb : 0, d < na ? d : na, lane, 0, [&](uint64_t x) {
+        return (A[x] ^ f) <= (B[d - 1 - x] ^ f);
+    });
+    return TileStart{a + i, b + (d - i), (uint32_t)p, (uint32_t)i, (uint32_t)(d - i), rel == 0 ? 1u : 0u};
 }
 
 // Count + stage: one workgroup per tile (tiles tile0 + blockIdx.x), no communication between
@@ -520,7 +553,7 @@ template <int NT, int K, int MAXSEG, bool BSR, bool COUNT_ONLY, bool GATHER, int
 __global__ __launch_bounds__(NT) void merge_tile_kernel(PairBatch in, TilePlan plan, TileOut out, uint32_t tile0)
 {
     static_assert(K >= 1 && K <= 32, "lane masks hold K bits");
-    static_assert(!DIRECT || (!GATHER && !BSR), "a direct tile is one plain CSR pair");
+    static_assert(!DIRECT || !GATHER, "a direct tile's units have a closed form");
     constexpr int U = NT * K;
     constexpr bool BLOCKP = LP != LP_MERGE;
     using Smem = MergeSmem<NT, K, MAXSEG, BSR, GATHER, BLOCKP>;
@@ -534,30 +567,63 @@ __global__ __launch_bounds__(NT) void merge_tile_kernel(PairBatch in, TilePlan p
         // ---- 1. descriptor and segment windows -------------------------------------------------
         // CSR: the tile's A and B runs load with its pair range (one round trip before the
         // staging is issued, not two)
-        // DIRECT (one pair in one tile, CSR form, the launch for plan.direct): the tile is the whole
-        // pair and nothing planned it, so its runs, its one segment and the error word come from the
-        // plan's fields here.  A template flag: a runtime branch here costs the batch tiles 3-5%.
+        // DIRECT (the launch for plan.direct: CSR batches and single pairs of few tiles): nothing
+        // planned the tiles.  Where the tile starts and where the next one does -- the pair of that
+        // unit, whose units have a closed form, and the merge-path split in it -- two waves find by
+        // 64-way searches, five dependent rounds for batches of up to 4,096 pairs; a plan launch and
+        // a split launch (a thread per tile, up to 30 dependent loads) cost a small batch 9 us and the
+        // two gaps.  A pair that is one tile starts and ends with it.  A template flag: a runtime
+        // branch here costs the batch tiles 3-5%.
         constexpr bool direct = DIRECT;
+        __shared__ TileStart edge[DIRECT ? 2 : 1];
         uint64_t ga0 = 0, ga1 = 0, gb0 = 0, gb1 = 0;
-        if constexpr (!GATHER) {
-            if constexpr (direct) {
+        uint32_t p_first = 0, p_last = 0;
+        TileEdges edges{};
+        if constexpr (direct) {
+            if (t == 0 && tid == 0 && out.error) *out.error = 0;  // before thread 0's own flags below
+            if (plan.single && plan.ntiles == 1) {
                 ga1 = plan.single_na;
                 gb1 = plan.single_nb;
-                if (tid == 0 && out.error) *out.error = 0;  // before thread 0's own flags below
+                edges.next_first = ~0u;
             } else {
+                const uint32_t w_ = tid / kWave;
+                if (w_ < 2) {
+                    const uint64_t v = min((uint64_t)(t + w_) * U, plan.utotal);
+                    const TileStart ts = tile_start(in, plan, v, lane_id());
+                    if (lane_id() == 0) edge[w_] = ts;
+                }
+                __syncthreads();
+                p_first = edge[0].pair;
+                p_last = edge[1].pair - (edge[1].at_start ? 1u : 0u);
+                ga0 = edge[0].ga;
+                gb0 = edge[0].gb;
+                ga1 = edge[1].ga;
+                gb1 = edge[1].gb;
+                edges = TileEdges{edge[0].sa, edge[0].sb, t + 1 < plan.ntiles ? edge[1].pair : ~0u, edge[1].sa, edge[1].sb};
+                if (tid == 0) {  // the maps that the placement reads
+                    plan.tile_first[t] = p_first;
+                    plan.tile_last[t] = p_last;
+                }
+            }
+        } else {
+            if constexpr (!GATHER) {
                 ga0 = plan.tile_ga[t];
                 ga1 = plan.tile_ga[t + 1];
                 gb0 = plan.tile_gb[t];
                 gb1 = plan.tile_gb[t + 1];
             }
+            p_first = plan.tile_first[t];
+            p_last = plan.tile_last[t];
         }
-        const uint32_t p_first = direct ? 0u : plan.tile_first[t], p_last = direct ? 0u : plan.tile_last[t];
         const uint64_t u0 = (uint64_t)t * U;
         uint32_t ulen = (uint32_t)((u0 + U < plan.utotal) ? U : plan.utotal - u0);
         uint32_t nseg = p_last - p_first + 1;
         bool bad = p_last < p_first || nseg > (uint32_t)MAXSEG || p_last >= in.P;
         if (bad) nseg = 0;
-        if (t == 0 && tid == 0 && out.error && !direct && plan.uoff[in.P] != plan.utotal) atomicOr(out.error, 4u);
+        if (t == 0 && tid == 0 && out.error && !plan.single &&
+            (direct ? in.a_end[in.P - 1] - in.a_beg[0] + in.b_end[in.P - 1] - in.b_beg[0] + (uint64_t)plan.c0 * in.P
+                    : plan.uoff[in.P]) != plan.utotal)
+            atomicOr(out.error, 4u);
         SegWin w{};
         uint32_t staged_words = 0;  // words loaded straight into LDS (flipped in place for int32 sets)
         uint32_t bstart = 0;        // key index where the staged B words start
@@ -584,7 +650,24 @@ __global__ __launch_bounds__(NT) void merge_tile_kernel(PairBatch in, TilePlan p
                     stage_run_lds<NT>(in.Bs, in.b_pool, gb0 & ~3ull, cB, sm.st + boff);
                 }
             }
-            if (tid < nseg) w = direct ? direct_window<false>(plan) : seg_window(in, plan, t, p_first, nseg, tid, ulen);
+            if (tid < nseg) {
+                if constexpr (direct) {
+                    SegRaw r{0, plan.single_na, 0, plan.single_nb, 0, plan.utotal};
+                    if (!plan.single) {
+                        const uint64_t p = (uint64_t)p_first + tid;
+                        r.a = in.a_beg[p];
+                        r.a1 = in.a_end[p];
+                        r.b = in.b_beg[p];
+                        r.b1 = in.b_end[p];
+                        r.u = csr_unit(in, plan.c0, p);
+                        r.u1 = r.u + (r.a1 - r.a) + (r.b1 - r.b) + plan.c0;
+                    }
+                    w = seg_window(plan, r, t, p_first, nseg, tid, ulen, edges);
+                    if (w.flags & 1u) plan.uoff[(uint64_t)p_first + tid] = r.u;  // for the placement
+                } else {
+                    w = seg_window(in, plan, t, p_first, nseg, tid, ulen);
+                }
+            }
             if (tid < nseg) {
                 sm.seg_la[tid] = shift_a + (uint32_t)(w.a + w.i0 - ga0);
                 sm.seg_lb[tid] = boff + shift_b + (uint32_t)(w.b + w.j0 - gb0);
@@ -628,6 +711,10 @@ __global__ __launch_bounds__(NT) void merge_tile_kernel(PairBatch in, TilePlan p
             nseg = 0;
             ulen = 0;
             if (tid == 0 && out.error) atomicOr(out.error, 2u);
+            if (DIRECT && tid == 0) {  // flagged (again) by the placement
+                plan.tile_first[t] = 0;
+                plan.tile_last[t] = ~0u;
+            }
         }
         if (tid < nseg) {
             const uint32_t wb = (uint32_t)(w.j1 - w.j0);
@@ -648,7 +735,7 @@ __global__ __launch_bounds__(NT) void merge_tile_kernel(PairBatch in, TilePlan p
             }
         }
 
-        merge_tile_compute<NT, K, MAXSEG, BSR, COUNT_ONLY, GATHER, LP>(sm, plan, out, t, nseg, ulen, p_first,
+        merge_tile_compute<NT, K, MAXSEG, BSR, COUNT_ONLY, GATHER, LP, DIRECT>(sm, plan, out, t, nseg, ulen, p_first,
                                                                        in.sflip, staged_words, bstart);
     }
 }

@@ -461,9 +461,9 @@ __global__ __launch_bounds__(NT, 4) void search_tile_kernel(PairBatch in, TilePl
         bool bad = p_last < p_first || nseg > (uint32_t)MAXSEG || p_last >= in.P;
         if (bad) nseg = 0;
         if (t == 0 && tid == 0 && out.error && !direct && plan.uoff[in.P] != plan.utotal) atomicOr(out.error, 4u);
-        if (dbatch && tid == 0 && !bad) {  // the tile maps the placement reads
-            plan.tile_first[t] = p_first;
-            plan.tile_last[t] = p_last;
+        if (dbatch && tid == 0) {  // the tile maps the placement reads
+            plan.tile_first[t] = bad ? 0u : p_first;
+            plan.tile_last[t] = bad ? ~0u : p_last;
         }
         uint32_t seg_pu = 0;  // direct batch: the segment's pair's first unit
         uint32_t cp = 0;
@@ -478,7 +478,7 @@ __global__ __launch_bounds__(NT, 4) void search_tile_kernel(PairBatch in, TilePl
                 seg_pu = sm.pkey[2 * p];
                 w = search_direct_window(in, p, seg_pu, sm.pkey[2 * p + 1], u0, ulen);
             } else {
-                w = direct ? direct_window<true>(plan) : seg_window(in, plan, t, p_first, nseg, tid, ulen);
+                w = direct ? direct_window(plan) : seg_window(in, plan, t, p_first, nseg, tid, ulen);
             }
             swap = (w.nb < w.na) ? 1u : 0u;  // probes come from the smaller side
             gp = (swap ? w.b : w.a) + w.i0;
@@ -1012,7 +1012,7 @@ __global__ __launch_bounds__(NT, 4) void search_tile_kernel(PairBatch in, TilePl
                 if (dbatch) plan.uoff[p] = seg_pu;  // for the placement (no plan wrote it)
             }
             if (plan.one_tile && out.out_off) out.out_off[p] = c0v;  // every pair lies in the one tile
-            if (out.counts) {
+            if (out.counts && (!direct || plan.one_tile)) {  // else the placement writes them
                 if ((f & 3u) == 3u) out.counts[p] = c;
                 else if (c) atomicAdd(&out.counts[p], c);
             }

@@ -509,16 +509,15 @@ int device_unit_total(setops_hip_batch *h, uint64_t *utotal, uint64_t *small)
 }
 
 // Tile kernels run one workgroup per tile; batches of more than kMaxGrid tiles take several
-// launches (tile offset tile0).  A direct plan (one plain pair in one tile, set only by the
-// single-pair entries) launches the kernels' DIRECT form, which takes the pair from the plan's
-// fields instead of the tile maps.
+// launches (tile offset tile0).  A direct plan launches the kernels' DIRECT form, which finds its
+// tiles' pairs itself instead of reading the tile maps.
 template <int K, bool BSR, bool CO, bool GA, int LP>
 void launch_merge_t(setops_hip_batch *h, const TileOut &out, hipStream_t stream)
 {
-    if constexpr (!BSR && !GA) {
+    if constexpr (!GA) {
         if (h->plan.direct) {
-            hipLaunchKernelGGL((merge_tile_kernel<kNTM, K, kMaxSeg, BSR, CO, GA, LP, true>), dim3(1), dim3(kNTM), 0,
-                               stream, h->in, h->plan, out, 0u);
+            hipLaunchKernelGGL((merge_tile_kernel<kNTM, K, kMaxSeg, BSR, CO, GA, LP, true>),
+                               dim3((uint32_t)h->plan.ntiles), dim3(kNTM), 0, stream, h->in, h->plan, out, 0u);
             return;
         }
     }
@@ -603,7 +602,7 @@ int batch_enqueue(setops_hip_batch *h, const TileOut &out, bool count_only, hipS
                   std::pair<hipEvent_t, hipEvent_t> *ev)
 {
     // plan: unit prefix and tile maps, then tile starts (one pair over several tiles: both in one
-    // launch; one pair in one tile: none, the tile kernel takes the pair as it is)
+    // launch; direct plans: none, the tiles find their pairs themselves)
     const bool single_split = h->plan.single && !h->plan.direct;
     if (h->plan.direct) {
         // no plan launch
@@ -640,8 +639,8 @@ int batch_enqueue(setops_hip_batch *h, const TileOut &out, bool count_only, hipS
     // scan: with few tiles the placement kernel scans the tile counts itself; with few groups one
     // kernel (a workgroup adds the earlier groups' tile counts itself); otherwise group sums,
     // one-block scan of the group sums (writes the totals), per-group scan
-    const bool place = !count_only || out.out_off;
-    const int fused = (place && h->plan.ntiles <= kFuseScanTiles) ? 1 : 0;
+    const int fused = h->plan.ntiles <= kFuseScanTiles ? 1 : 0;
+    const bool place = fused || !count_only || out.out_off;
     if (!fused) {
         const uint32_t ngroups = (h->plan.ntiles + kScanGroup - 1) / kScanGroup;
         const int direct = ngroups <= kScanDirectGroups ? 1 : 0;
@@ -695,6 +694,35 @@ void graph_drop(setops_hip_batch *h)
     h->graph = nullptr;
 }
 
+// Whether a run needs no plan launch (plan.direct: the tile kernels' DIRECT form, over at most the
+// tiles that a fused placement scans) and whether its one tile's outputs are final (plan.one_tile:
+// plain sets, room for every result, the tile's slot is the output).
+//   merge policy: CSR batches and single pairs, whose units have a closed form (601 uneven pairs,
+//     128 tiles: 32 us a run with the plan and split launches, 22.5 us without; a pair of 2^16 + 2^16: 18 and
+//     12 us; beyond the fused placement's tiles the searches in every tile would cost more than
+//     the two launches);
+//   search policy: gather and CSR batches of at most kNT plain pairs (every tile scans their units),
+//     a single pair of one tile.
+void plan_direct(setops_hip_batch *h, bool count_only, uint64_t cap, bool totals)
+{
+    const TilePlan &pl = h->plan;
+    const bool few = pl.ntiles <= kFuseScanTiles, one = pl.ntiles == 1;
+    bool direct, final_ = one && !h->bsr;
+    if (pl.policy == POLICY_MERGE) {
+        direct = few && !h->gather;
+        // a pair has at most half its elements in common
+        final_ = final_ && direct && (pl.single ? totals : true) &&
+                 (count_only || cap >= (pl.single ? std::min(pl.single_na, pl.single_nb) : (pl.utotal - h->P * pl.c0) / 2));
+    } else if (pl.single) {
+        final_ = direct = final_ && totals && (count_only || cap >= std::min(pl.single_na, pl.single_nb));
+    } else {
+        final_ = final_ && !count_only && h->P <= (uint64_t)kMaxSeg && cap >= pl.utotal - h->P * pl.c0;
+        direct = few && !count_only && !h->bsr && h->P <= (uint64_t)kNT && (!one || final_);
+    }
+    h->plan.direct = direct ? 1u : 0u;
+    h->plan.one_tile = direct && final_ ? 1u : 0u;
+}
+
 // A run: eager when timed (events around the tile kernel), otherwise the launch sequence is
 // captured once into a HIP graph (per handle, per set of output pointers and plan) and replayed
 // with one launch.  The sequence records kernels only (no memset or copy nodes).
@@ -716,18 +744,7 @@ int batch_launch(setops_hip_batch *h, uint32_t *d_out, uint32_t *d_out_s, uint64
     out.error = h->d_error;
     // a run on another stream than the last one would share the workspace and staging with it
     if (h->ran && h->last_stream != stream) HIP_TRY(hipStreamSynchronize(h->last_stream));
-    // a plain search-policy batch of at most kNT pairs runs the search tile's direct form, which
-    // finds its pairs itself (no plan launch): in one tile with room for every probe's result, the
-    // tile's slot is the output and the tile writes the offsets and totals (no scan, no
-    // placement); over a few tiles (a fused placement follows), when no per-pair counts are asked
-    // for (they would be added up across tiles from zero, and nothing zeroes them)
-    if (!h->plan.single) {
-        const bool small = !count_only && !h->bsr && h->plan.policy == POLICY_SEARCH && h->P <= (uint64_t)kNT;
-        const bool one = h->plan.ntiles == 1 && h->P <= (uint64_t)kMaxSeg && cap >= h->plan.utotal - h->P * h->plan.c0;
-        const bool few = h->plan.ntiles > 1 && h->plan.ntiles <= kFuseScanTiles && d_counts == nullptr;
-        h->plan.direct = (small && (one || few)) ? 1u : 0u;
-    }
-    h->plan.one_tile = (h->plan.direct && h->plan.ntiles == 1) ? 1u : 0u;
+    plan_direct(h, count_only, cap, d_totals != nullptr);
     if (!count_only) {
         int rc = stage_reserve(h);
         if (rc != SETOPS_OK) return rc;
@@ -937,8 +954,6 @@ int single_launch(int algo, const uint32_t *dA, const uint32_t *dAs, size_t na, 
     h->in.nx = nx;
     h->plan.single_na = na;
     h->plan.single_nb = nb;
-    // one tile, plain sets, and room for any result: the tile writes the output and the totals
-    h->plan.direct = (h->plan.ntiles == 1 && !e->bsr && dTot && (dO == nullptr || cap >= std::min(na, nb))) ? 1u : 0u;
     return batch_launch(h, dO, dOs, cap, nullptr, nullptr, dTot, s);
 }
 
@@ -1007,9 +1022,8 @@ int noalloc_launch(int algo, const uint32_t *dA, const uint32_t *dAs, size_t na,
     h->in.contig = 1;
     h->in.sflip = sflip_of(algo);
     const bool count_only = (dO == nullptr && dOs == nullptr);
-    h->plan.direct = (ntiles == 1 && !e->bsr && (count_only || cap >= std::min(na, nb))) ? 1u : 0u;
-    h->plan.one_tile = h->plan.direct;
-    if (!count_only && h->plan.direct) h->plan.stage = dO;  // the one tile's slot is the output
+    plan_direct(h, count_only, cap, true);
+    if (!count_only && h->plan.one_tile) h->plan.stage = dO;  // the one tile's slot is the output
     TileOut out{};
     out.out = dO;
     out.out_s = dOs;
@@ -1463,11 +1477,7 @@ int setops_hip_batch_reserve(setops_hip_batch *handle, uint64_t npairs, uint64_t
         h->cap_pairs = cp;
         h->cap_tiles = ct;
     }
-    const uint32_t *keep = h->plan.stage;
-    int rc = stage_grow(h, ntiles);
-    if (rc != SETOPS_OK) return rc;
-    if (h->plan.direct) h->plan.stage = const_cast<uint32_t *>(keep);
-    return SETOPS_OK;
+    return stage_grow(h, ntiles);  // (the plan's staging pointer is set by every run that writes results)
 }
 
 int setops_hip_batch_step(setops_hip_batch *handle, const uint64_t *h_idx, uint64_t *d_idx, uint64_t npairs,

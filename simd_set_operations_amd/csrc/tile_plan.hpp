@@ -104,12 +104,12 @@ struct TilePlan {
     uint32_t single;
     uint64_t *single_off;
     uint64_t single_na, single_nb;
-    // single pair in one tile, plain sets, output capacity >= min(na, nb): `stage` is the caller's
-    // output, the tile kernel writes the totals, and the split, scan and placement are skipped
+    // the tile kernels' DIRECT form runs: no plan launch, every tile finds its pairs (and, merge
+    // policy, its splits) itself, and a fused placement writes the per-pair counts
     uint32_t direct;
-    // the one tile's outputs are final (a direct plan, or a plain search-policy batch of one tile
-    // with output room for every unit): `stage` is the caller's output and the search tile writes
-    // the per-pair offsets and the totals; the scan and placement are skipped
+    // a direct plan of one tile of plain sets with output room for every result: the tile's outputs
+    // are final, `stage` is the caller's output, the tile writes the per-pair offsets, the counts
+    // and the totals, and the placement is skipped
     uint32_t one_tile;
 };
 
@@ -611,20 +611,30 @@ constexpr uint32_t kFuseScanTiles = 1024;
 template <int NT, int Q, bool BSR, bool FUSED>
 __global__ __launch_bounds__(NT) void place_tiles_kernel(PairBatch in, TilePlan plan, TileOut out, uint32_t tile0)
 {
-    __shared__ unsigned long long red[FUSED ? NT / kWave : 1][2];
     const uint32_t tid = threadIdx.x;
     const uint64_t t = (uint64_t)tile0 + blockIdx.x;
     if (t >= plan.ntiles) return;
     const uint32_t sw = plan.stage_words;
     const uint64_t pf = plan.tile_first[t];
     uint64_t pl = plan.tile_last[t];
-    if (pl >= in.P) pl = in.P - 1;  // stale maps (flagged by the tile kernel): stay inside the pairs
+    if (pl >= in.P) {
+        // stale maps (flagged by the tile kernel; the tiles of a direct plan, which race with the one
+        // that clears the flags, leave it to this kernel): stay inside the pairs
+        if (FUSED && plan.direct && tid == 0 && out.error) atomicOr(out.error, 2u);
+        pl = in.P - 1;
+    }
     uint64_t base;
     uint32_t n;
+    const bool pair_counts = FUSED && plan.direct && out.counts;
+    uint32_t t2 = plan.ntiles, later = 0;
     if constexpr (FUSED) {
         // results before the tile (and, for the last tile, the elements of every tile)
         const bool last = t + 1 == plan.ntiles;
         unsigned long long b = 0, el = 0;
+        // with a direct plan the per-pair counts are written here: where the tile's last pair goes on
+        // into later tiles, its results are those of the tiles up to the one (t2) where the next pair
+        // starts, and those before that pair there
+        if (pair_counts && pl + 1 < in.P) t2 = (uint32_t)tile_of_unit(plan.uoff[pl + 1], plan.U, 1.0 / (double)plan.U);
         // four counts per load, every load in flight together (tile arrays are padded to 256 bytes)
         constexpr int QF = (int)kFuseScanTiles / (4 * NT);
         static_assert(QF * 4 * NT == (int)kFuseScanTiles, "whole 16-byte loads cover the fused tile limit");
@@ -645,6 +655,7 @@ __global__ __launch_bounds__(NT) void place_tiles_kernel(PairBatch in, TilePlan 
 #pragma unroll
                 for (uint32_t j = 0; j < 4; j++) {
                     if (i + j < t) b += cw[j];
+                    if (i + j > t && i + j < t2 && i + j < plan.ntiles) later += cw[j];
                     if (last && i + j < plan.ntiles) {
                         const uint32_t ew[4] = {ev[q].x, ev[q].y, ev[q].z, ev[q].w};
                         el += ew[j];
@@ -656,18 +667,10 @@ __global__ __launch_bounds__(NT) void place_tiles_kernel(PairBatch in, TilePlan 
         for (int d = 1; d < kWave; d <<= 1) {
             b += __shfl_xor(b, d, kWave);
             el += __shfl_xor(el, d, kWave);
+            later += __shfl_xor(later, d, kWave);
         }
-        if (lane_id() == 0) {
-            red[tid / kWave][0] = b;
-            red[tid / kWave][1] = el;
-        }
-        __syncthreads();
-        base = 0;
-        el = 0;
-        for (int k = 0; k < NT / kWave; k++) {
-            base += red[k][0];
-            el += red[k][1];
-        }
+        static_assert(NT == kWave, "one wave sums the counts");
+        base = b;
         n = plan.tile_count[t];
         if (tid == 0) {
             plan.tile_off[t] = base;
@@ -692,10 +695,15 @@ __global__ __launch_bounds__(NT) void place_tiles_kernel(PairBatch in, TilePlan 
     const uint64_t p0 = pf + tid;
     uint64_t up = 0;
     uint32_t ploc = 0;
-    if (out.out_off && p0 <= pl) {
+    if ((out.out_off || pair_counts) && p0 <= pl) {
         up = plan.uoff[p0];
         ploc = plan.pair_local[p0];
     }
+    // the result offset, from the tile's first result, of pair p's end (p starts in the tile)
+    auto pair_end = [&](uint64_t p) {
+        if (p < pl) return plan.pair_local[p + 1];
+        return n + later + (pl + 1 < in.P ? plan.pair_local[pl + 1] : 0u);
+    };
     if (out.out) {
         const uint64_t room = out.cap > base ? out.cap - base : 0;
         const uint32_t lim = (uint64_t)n < room ? n : (uint32_t)room;
@@ -722,12 +730,18 @@ __global__ __launch_bounds__(NT) void place_tiles_kernel(PairBatch in, TilePlan 
             }
         }
     }
-    if (out.out_off) {
-        if (p0 <= pl && up >= u0) out.out_off[p0] = base + ploc;
+    if (out.out_off || pair_counts) {
+        if (p0 <= pl && up >= u0) {
+            if (out.out_off) out.out_off[p0] = base + ploc;
+            if (pair_counts) out.counts[p0] = pair_end(p0) - ploc;
+        }
         for (uint64_t p = p0 + NT; p <= pl; p += NT) {  // tiles of more than NT pairs
             const uint64_t uq = plan.uoff[p];
             const uint32_t lq = plan.pair_local[p];
-            if (uq >= u0) out.out_off[p] = base + lq;
+            if (uq >= u0) {
+                if (out.out_off) out.out_off[p] = base + lq;
+                if (pair_counts) out.counts[p] = pair_end(p) - lq;
+            }
         }
     }
 }
@@ -766,19 +780,30 @@ __device__ __forceinline__ TileEdges tile_edges(const TilePlan &plan, uint32_t t
     return e;
 }
 
+// The bounds and units of one segment's pair.
+struct SegRaw {
+    uint64_t a, a1, b, b1, u, u1;
+};
+
+// First unit of pair p of a CSR batch under the merge policy (p == P: the unit total).
+__device__ __forceinline__ uint64_t csr_unit(const PairBatch &in, uint32_t c0, uint64_t p)
+{
+    return in.a_beg[p] - in.a_beg[0] + in.b_beg[p] - in.b_beg[0] + (uint64_t)c0 * p;
+}
+
 // Window of segment s of tile t (pairs p_first .. p_last); the last segment ends where the next
 // tile starts if that tile starts in the same pair, else at the pair's end.
-__device__ __forceinline__ SegWin seg_window(const PairBatch &in, const TilePlan &plan, uint32_t t, uint32_t p_first,
+__device__ __forceinline__ SegWin seg_window(const TilePlan &plan, const SegRaw &r, uint32_t t, uint32_t p_first,
                                              uint32_t nseg, uint32_t s, uint32_t ulen, const TileEdges &e)
 {
     SegWin w;
     const uint64_t p = (uint64_t)p_first + s;
     w.p = p;
-    w.a = in.a_beg[p];
-    w.b = in.b_beg[p];
-    w.na = in.a_end[p] - w.a;
-    w.nb = in.b_end[p] - w.b;
-    const uint64_t up = plan.uoff[p], upn = plan.uoff[p + 1];
+    w.a = r.a;
+    w.b = r.b;
+    w.na = r.a1 - r.a;
+    w.nb = r.b1 - r.b;
+    const uint64_t up = r.u, upn = r.u1;
     const uint64_t u0 = (uint64_t)t * plan.U;
     w.i0 = (s == 0) ? e.sa : 0;
     w.j0 = (s == 0) ? e.sb : 0;
@@ -800,30 +825,25 @@ __device__ __forceinline__ SegWin seg_window(const PairBatch &in, const TilePlan
 __device__ __forceinline__ SegWin seg_window(const PairBatch &in, const TilePlan &plan, uint32_t t, uint32_t p_first,
                                              uint32_t nseg, uint32_t s, uint32_t ulen)
 {
-    return seg_window(in, plan, t, p_first, nseg, s, ulen, tile_edges(plan, t));
+    const uint64_t p = (uint64_t)p_first + s;
+    const SegRaw r{in.a_beg[p], in.a_end[p], in.b_beg[p], in.b_end[p], plan.uoff[p], plan.uoff[p + 1]};
+    return seg_window(plan, r, t, p_first, nseg, s, ulen, tile_edges(plan, t));
 }
 
-// The one segment of a direct plan (one pair in one tile): the whole pair, starting and ending
-// in the tile at unit 0 (what seg_window gives for it under the tile kind's policy).
-template <bool SEARCH>
+// The one segment of a direct search plan of a single pair: the whole pair, starting and ending in the
+// tile at unit 0 (what seg_window gives for it).
 __device__ __forceinline__ SegWin direct_window(const TilePlan &plan)
 {
     SegWin w;
-    const uint64_t na = plan.single_na, nb = plan.single_nb;
     w.p = 0;
     w.a = 0;
     w.b = 0;
-    w.na = na;
-    w.nb = nb;
+    w.na = plan.single_na;
+    w.nb = plan.single_nb;
     w.i0 = 0;
     w.j0 = 0;
-    if constexpr (SEARCH) {
-        w.i1 = na < nb ? na : nb;
-        w.j1 = 0;
-    } else {
-        w.i1 = na;
-        w.j1 = nb;
-    }
+    w.i1 = min(w.na, w.nb);
+    w.j1 = 0;
     w.u = 0;
     w.flags = 3u;
     return w;
