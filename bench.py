@@ -4,7 +4,7 @@
 Workload (the batched configuration of this path): 65,536 pairs of sorted unique u32; larger
 size log-uniform in [2^6, 2^14]; smaller = larger / r, r log-uniform in [1, 1024]; element space
 10 x larger; selectivity ~ U[0,1] with shared elements planted first.  One step = one batch
-intersection (plan, split, tile, scan and placement kernels, replayed as one HIP graph) producing
+intersection (plan, split, tile, scan and placement kernels) producing
 per-pair counts, per-pair offsets and the compacted results, with the inputs already resident in
 HBM.
 

@@ -53,7 +53,7 @@ def time_entry(torch, algo, A, a_off, B, b_off, shared, runs):
         _, cnt, _ = db.results()
         if not np.all(cnt == shared):
             raise RuntimeError(f"{algo}: per-pair counts differ from the planted {shared}")
-        for _ in range(2):  # the replayed launch graph
+        for _ in range(2):  # the first runs
             db.run(stream)
         e0 = torch.cuda.Event(enable_timing=True)
         e1 = torch.cuda.Event(enable_timing=True)

@@ -268,18 +268,6 @@ struct setops_hip_batch {
     hipStream_t last_stream = nullptr;  // the stream of the last run (NULL: the HIP null stream)
     bool ran = false;                   // a run was enqueued (on last_stream)
     bool timing = false;
-    // captured launch sequence (batch_launch)
-    bool use_graph = true;
-    hipStream_t cap_stream = nullptr;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t graph_exec = nullptr;
-    struct GraphKeyT {
-        void *out, *out_s;
-        uint64_t cap;
-        void *out_off, *counts, *totals;
-        PairBatch in;
-        TilePlan plan;
-    } graph_key{}, seen_key{};
     std::vector<std::pair<hipEvent_t, hipEvent_t>> events;  // pending timed runs
     std::vector<std::pair<hipEvent_t, hipEvent_t>> spare;
 };
@@ -686,14 +674,6 @@ int batch_enqueue(setops_hip_batch *h, const TileOut &out, bool count_only, hipS
     return SETOPS_OK;
 }
 
-void graph_drop(setops_hip_batch *h)
-{
-    if (h->graph_exec) (void)hipGraphExecDestroy(h->graph_exec);
-    if (h->graph) (void)hipGraphDestroy(h->graph);
-    h->graph_exec = nullptr;
-    h->graph = nullptr;
-}
-
 // Whether a run needs no plan launch (plan.direct: the tile kernels' DIRECT form, over at most the
 // tiles that a fused placement scans) and whether its one tile's outputs are final (plan.one_tile:
 // plain sets, room for every result, the tile's slot is the output).
@@ -723,9 +703,10 @@ void plan_direct(setops_hip_batch *h, bool count_only, uint64_t cap, bool totals
     h->plan.one_tile = direct && final_ ? 1u : 0u;
 }
 
-// A run: eager when timed (events around the tile kernel), otherwise the launch sequence is
-// captured once into a HIP graph (per handle, per set of output pointers and plan) and replayed
-// with one launch.  The sequence records kernels only (no memset or copy nodes).
+// A run: the launch sequence, enqueued kernel by kernel.  (Captured once and replayed as a HIP graph,
+// a run of two to nine kernels costs 4 to 6 us more: 601 uneven pairs, two kernels, 22.8 against
+// 18.3 us; a request-loop step, two kernels and three copies, 73 against 57.6; 65,536 uneven
+// pairs, five kernels, 255.2 against 250.9; the resident set, three kernels, 57.9 against 52.7.)
 int batch_launch(setops_hip_batch *h, uint32_t *d_out, uint32_t *d_out_s, uint64_t cap, uint64_t *d_out_off,
                  uint32_t *d_counts, unsigned long long *d_totals, hipStream_t stream)
 {
@@ -752,57 +733,19 @@ int batch_launch(setops_hip_batch *h, uint32_t *d_out, uint32_t *d_out_s, uint64
     }
     h->last_stream = stream;
     h->ran = true;
-    if (h->timing || !h->use_graph) {
-        std::pair<hipEvent_t, hipEvent_t> ev{nullptr, nullptr};
-        if (h->timing) {
-            if (!h->spare.empty()) {
-                ev = h->spare.back();
-                h->spare.pop_back();
-            } else {
-                HIP_TRY(hipEventCreate(&ev.first));
-                HIP_TRY(hipEventCreate(&ev.second));
-            }
+    std::pair<hipEvent_t, hipEvent_t> ev{nullptr, nullptr};
+    if (h->timing) {
+        if (!h->spare.empty()) {
+            ev = h->spare.back();
+            h->spare.pop_back();
+        } else {
+            HIP_TRY(hipEventCreate(&ev.first));
+            HIP_TRY(hipEventCreate(&ev.second));
         }
-        int rc = batch_enqueue(h, out, count_only, stream, h->timing ? &ev : nullptr);
-        if (h->timing) h->events.push_back(ev);
-        return rc;
     }
-    // the captured sequence depends on the outputs and on everything the plan holds
-    setops_hip_batch::GraphKeyT key;
-    std::memset(static_cast<void *>(&key), 0, sizeof key);
-    key.out = d_out;
-    key.out_s = d_out_s;
-    key.cap = out.cap;
-    key.out_off = d_out_off;
-    key.counts = d_counts;
-    key.totals = d_totals;
-    key.in = h->in;
-    key.plan = h->plan;
-    const bool cached = h->graph_exec && std::memcmp(&key, &h->graph_key, sizeof key) == 0;
-    if (!cached && std::memcmp(&key, &h->seen_key, sizeof key) != 0) {
-        // first run with these arguments: eager (a run whose arguments change every time, like a
-        // rebound serving batch or a single pair, never pays for a capture)
-        h->seen_key = key;
-        return batch_enqueue(h, out, count_only, stream, nullptr);
-    }
-    if (!cached) {
-        graph_drop(h);
-        if (!h->cap_stream) HIP_TRY(hipStreamCreateWithFlags(&h->cap_stream, hipStreamNonBlocking));
-        HIP_TRY(hipStreamBeginCapture(h->cap_stream, hipStreamCaptureModeThreadLocal));
-        const int rc = batch_enqueue(h, out, count_only, h->cap_stream, nullptr);
-        hipGraph_t g = nullptr;
-        const hipError_t e = hipStreamEndCapture(h->cap_stream, &g);
-        if (rc != SETOPS_OK) {
-            if (g) (void)hipGraphDestroy(g);
-            return rc;
-        }
-        if (e != hipSuccess) return fail(SETOPS_ERR_HIP, "hipStreamEndCapture failed: %s", hipGetErrorString(e));
-        h->graph = g;
-        HIP_TRY(hipGraphInstantiate(&h->graph_exec, g, nullptr, nullptr, 0));
-        h->graph_key = key;
-    }
-    HIP_TRY(hipGraphLaunch(h->graph_exec, stream));
-    return SETOPS_OK;
+    const int rc = batch_enqueue(h, out, count_only, stream, h->timing ? &ev : nullptr);
+    if (h->timing) h->events.push_back(ev);
+    return rc;
 }
 
 // Shared by the CSR and gather constructors: a_end == NULL means CSR (a_end = a_beg + 1).
@@ -883,8 +826,6 @@ void batch_free(setops_hip_batch *h)
         (void)hipEventDestroy(e.first);
         (void)hipEventDestroy(e.second);
     }
-    graph_drop(h);
-    if (h->cap_stream) (void)hipStreamDestroy(h->cap_stream);
     if (h->ws) (void)hipFree(h->ws);
     if (h->stage) (void)hipFree(h->stage);
     if (h->b_idx) (void)hipFree(h->b_idx);
@@ -988,7 +929,6 @@ int noalloc_launch(int algo, const uint32_t *dA, const uint32_t *dAs, size_t na,
     h->gather = false;
     h->P = 1;
     h->timing = false;
-    h->use_graph = false;
     h->in = PairBatch{};
     h->plan = TilePlan{};
     const uint64_t U = units_per_tile(e->kind, e->bsr, h->shape);
@@ -1464,8 +1404,7 @@ int setops_hip_batch_reserve(setops_hip_batch *handle, uint64_t npairs, uint64_t
     const uint64_t ntiles = std::max<uint64_t>(1, (units + pad * std::max<uint64_t>(npairs, 1) + U - 1) / U);
     if (ntiles >= 0x7FFFFFFFull) return fail(SETOPS_ERR_INVALID, "too many units: %llu", (unsigned long long)units);
     if (!h->ws || npairs > h->cap_pairs || ntiles > h->cap_tiles) {
-        // ws_layout repoints the plan's arrays; every run rewrites them, and a cached launch graph
-        // keyed on the old pointers is not replayed
+        // ws_layout repoints the plan's arrays; every run rewrites them
         if (h->ws) {
             if (h->ran) HIP_TRY(hipStreamSynchronize(h->last_stream));
             HIP_TRY(hipFree(h->ws));
