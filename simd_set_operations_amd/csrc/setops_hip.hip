@@ -151,6 +151,12 @@ struct Context {
     int num_cu = 0;
     hipStream_t stream = nullptr;
     std::mutex host_mu;  // serialises the host-pointer entry points
+    // pinned host memory mapped for the device (kPinIn + kPinOut bytes and the totals), for the
+    // host-pointer entry points: inputs on their way to the device, results on their way back
+    char *pin = nullptr;
+    char *pin_dev = nullptr;
+    bool pin_tried = false;
+    hipEvent_t pin_done = nullptr;
     // grow-only device buffers for the host-pointer entry points
     void *host_buf = nullptr;
     size_t host_buf_bytes = 0;
@@ -973,6 +979,132 @@ int noalloc_launch(int algo, const uint32_t *dA, const uint32_t *dAs, size_t na,
     return batch_enqueue(h, out, count_only, s, nullptr);
 }
 
+// ---- host-pointer calls: inputs and results through pinned memory ------------------------------------
+// A call's inputs are copied once by the CPU into pinned memory that the device sees: short ones
+// (kMapIn) the kernels read there, over the bus, longer ones (kPinIn) a copy kernel moves to the
+// device, in the same queue as the tiles.  Results (kPinOut) and totals are written by the kernels
+// into that memory, so that a call waits once, for its kernels, and copies its result out.  (A copy of
+// the runtime costs 8 to 15 us, whatever its size: with two uploads, the totals and the result a pair
+// of 1,000 + 1,300 took 50 us, 24 now; a k-set query of 5 sets of up to 2^18, 16 copies, 311 us, 171
+// now.  Up to kMapIn the copy kernel costs more than reading over the bus: 84 KB 33 against 30.5 us, 107
+// KB 33.5 against 33.8.)  Larger inputs and results go by the runtime's copies.
+constexpr size_t kMapIn = 96u << 10;
+constexpr size_t kPinIn = 4u << 20;
+constexpr size_t kPinOut = 2u << 20;
+
+__global__ __launch_bounds__(256) void copy_chunks_kernel(const uint4 *__restrict__ src, uint4 *__restrict__ dst,
+                                                          uint32_t n)
+{
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < n; i += gridDim.x * 256u) dst[i] = src[i];
+}
+
+// Allocates the pinned memory on first use; false if there is none (the calls then do without).
+bool have_pin()
+{
+    if (!g_ctx.pin_tried) {
+        g_ctx.pin_tried = true;
+        void *p = nullptr, *d = nullptr;
+        if (hipHostMalloc(&p, kPinIn + kPinOut + 256, hipHostMallocMapped) != hipSuccess) {
+            (void)hipGetLastError();
+        } else if (hipHostGetDevicePointer(&d, p, 0) != hipSuccess || !d) {
+            (void)hipGetLastError();
+            (void)hipHostFree(p);
+        } else {
+            g_ctx.pin = static_cast<char *>(p);
+            g_ctx.pin_dev = static_cast<char *>(d);
+        }
+    }
+    return g_ctx.pin != nullptr;
+}
+
+// The inputs of one call: `bytes` of device memory at dev (256-byte aligned pieces, put() in order);
+// with pinned memory and room in it they pass through there.
+struct HostInputs {
+    char *dev;
+    size_t used = 0, sent = 0;
+    bool pinned, mapped;
+    HostInputs(char *d, size_t bytes, bool may_map)
+        : dev(d), pinned(bytes <= kPinIn && have_pin()), mapped(pinned && may_map && bytes <= kMapIn)
+    {
+    }
+    // Where the device finds the n words of src once send() has returned.
+    const uint32_t *put(const uint32_t *src, size_t n, hipStream_t s, int *rc)
+    {
+        const size_t at = used;
+        used += align_up(n * 4 + 16, 256);
+        if (pinned) {
+            if (n) std::memcpy(g_ctx.pin + at, src, n * 4);
+            return reinterpret_cast<const uint32_t *>((mapped ? g_ctx.pin_dev : dev) + at);
+        }
+        if (n && *rc == SETOPS_OK) {
+            const hipError_t e = hipMemcpyAsync(dev + at, src, n * 4, hipMemcpyHostToDevice, s);
+            if (e != hipSuccess) *rc = fail(SETOPS_ERR_HIP, "hipMemcpyAsync failed: %s", hipGetErrorString(e));
+        }
+        return reinterpret_cast<const uint32_t *>(dev + at);
+    }
+    // Enqueues the move of what was put since the last send.
+    int send(hipStream_t s)
+    {
+        if (pinned && !mapped && used > sent) {
+            const uint32_t n = (uint32_t)((used - sent) / 16);
+            hipLaunchKernelGGL(copy_chunks_kernel, dim3(std::min<uint32_t>((n + 255) / 256, 512u)), dim3(256), 0, s,
+                               reinterpret_cast<const uint4 *>(g_ctx.pin_dev + sent),
+                               reinterpret_cast<uint4 *>(dev + sent), n);
+            HIP_TRY(hipGetLastError());
+        }
+        sent = used;
+        return SETOPS_OK;
+    }
+};
+
+// A call's results and totals: in pinned memory where there is room, else at dev (two pieces of
+// piece_bytes, the second for BSR states, and 256 bytes for the totals).
+struct HostResults {
+    uint32_t *out[2];
+    unsigned long long *tot;
+    bool pinned;
+    HostResults(char *dev, size_t piece_bytes, int pieces) : pinned(have_pin() && pieces * piece_bytes <= kPinOut)
+    {
+        char *p = pinned ? g_ctx.pin_dev + kPinIn : dev;
+        out[0] = reinterpret_cast<uint32_t *>(p);
+        out[1] = reinterpret_cast<uint32_t *>(p + piece_bytes);
+        step = piece_bytes;
+        // (totals in pinned memory whenever there is any)
+        tot = reinterpret_cast<unsigned long long *>(have_pin() ? g_ctx.pin_dev + kPinIn + kPinOut : dev + 2 * piece_bytes);
+    }
+    // Marks where the totals are written, for a wait that does not wait for what is enqueued later.
+    int mark(hipStream_t s)
+    {
+        if (!g_ctx.pin) return SETOPS_OK;
+        if (!g_ctx.pin_done) HIP_TRY(hipEventCreateWithFlags(&g_ctx.pin_done, hipEventDisableTiming));
+        HIP_TRY(hipEventRecord(g_ctx.pin_done, s));
+        marked = true;
+        return SETOPS_OK;
+    }
+    // Waits for the mark, or the stream, and reads the totals.
+    int wait(hipStream_t s, unsigned long long *t)
+    {
+        if (!g_ctx.pin) HIP_TRY(hipMemcpyAsync(t, tot, 16, hipMemcpyDeviceToHost, s));
+        if (marked) HIP_TRY(hipEventSynchronize(g_ctx.pin_done));
+        else HIP_TRY(hipStreamSynchronize(s));
+        marked = false;
+        if (g_ctx.pin) std::memcpy(t, g_ctx.pin + kPinIn + kPinOut, 16);
+        return SETOPS_OK;
+    }
+    // Copies n words of piece i out (after wait).
+    int get(int i, uint32_t *dst, size_t n) const
+    {
+        if (!n) return SETOPS_OK;
+        if (pinned) std::memcpy(dst, g_ctx.pin + kPinIn + i * step, n * 4);
+        else HIP_TRY(hipMemcpy(dst, out[i], n * 4, hipMemcpyDeviceToHost));
+        return SETOPS_OK;
+    }
+
+private:
+    size_t step;
+    bool marked = false;
+};
+
 // One pair, host pointers: upload, run, download.  keys/states of each side.
 int run_single_pair(int algo, const uint32_t *a, const uint32_t *as, size_t na, const uint32_t *b,
                     const uint32_t *bs, size_t nb, uint32_t *out, uint32_t *out_s, size_t out_cap, size_t *out_len,
@@ -980,57 +1112,84 @@ int run_single_pair(int algo, const uint32_t *a, const uint32_t *as, size_t na, 
 {
     const AlgoEntry *e = algo_entry(algo);
     const bool count_only = (out == nullptr && out_s == nullptr);
-    const size_t bytes_a = align_up(na * 4 + 16, 256), bytes_b = align_up(nb * 4 + 16, 256);
     const size_t cap = std::min(na, nb);
     const size_t bytes_o = align_up(cap * 4 + 16, 256);
-    const int mult = e->bsr ? 2 : 1;
-    const size_t bytes = mult * (bytes_a + bytes_b + bytes_o) + 256;
+    const size_t bytes_in = (e->bsr ? 2 : 1) * (align_up(na * 4 + 16, 256) + align_up(nb * 4 + 16, 256));
     void *buf = nullptr;
-    int rc = host_scratch(bytes, &buf);
+    int rc = host_scratch(bytes_in + 2 * bytes_o + 256, &buf);
     if (rc != SETOPS_OK) return rc;
-    char *p = static_cast<char *>(buf);
-    uint32_t *dA = reinterpret_cast<uint32_t *>(p);
-    p += bytes_a;
-    uint32_t *dB = reinterpret_cast<uint32_t *>(p);
-    p += bytes_b;
-    uint32_t *dO = reinterpret_cast<uint32_t *>(p);
-    p += bytes_o;
-    uint32_t *dAs = nullptr, *dBs = nullptr, *dOs = nullptr;
-    if (e->bsr) {
-        dAs = reinterpret_cast<uint32_t *>(p);
-        p += bytes_a;
-        dBs = reinterpret_cast<uint32_t *>(p);
-        p += bytes_b;
-        dOs = reinterpret_cast<uint32_t *>(p);
-        p += bytes_o;
-    }
-    unsigned long long *dTot = reinterpret_cast<unsigned long long *>(p);
     hipStream_t s = g_ctx.stream;
-    if (na) HIP_TRY(hipMemcpyAsync(dA, a, na * 4, hipMemcpyHostToDevice, s));
-    if (nb) HIP_TRY(hipMemcpyAsync(dB, b, nb * 4, hipMemcpyHostToDevice, s));
+    HostInputs in(static_cast<char *>(buf), bytes_in, true);
+    HostResults res(static_cast<char *>(buf) + bytes_in, bytes_o, e->bsr ? 2 : 1);
+    const uint32_t *dA = in.put(a, na, s, &rc), *dB = in.put(b, nb, s, &rc), *dAs = nullptr, *dBs = nullptr;
     if (e->bsr) {
-        if (na) HIP_TRY(hipMemcpyAsync(dAs, as, na * 4, hipMemcpyHostToDevice, s));
-        if (nb) HIP_TRY(hipMemcpyAsync(dBs, bs, nb * 4, hipMemcpyHostToDevice, s));
+        dAs = in.put(as, na, s, &rc);
+        dBs = in.put(bs, nb, s, &rc);
     }
-    rc = single_launch(algo, dA, dAs, na, dB, dBs, nb, count_only ? nullptr : dO, count_only ? nullptr : dOs, cap,
-                       dTot, s);
+    if (rc == SETOPS_OK) rc = in.send(s);
+    if (rc != SETOPS_OK) return rc;
+    rc = single_launch(algo, dA, dAs, na, dB, dBs, nb, count_only ? nullptr : res.out[0],
+                       count_only || !e->bsr ? nullptr : res.out[1], cap, res.tot, s);
     if (rc != SETOPS_OK) return rc;
     unsigned long long tot[2] = {0, 0};
-    HIP_TRY(hipMemcpyAsync(tot, dTot, sizeof tot, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    rc = res.wait(s, tot);
+    if (rc != SETOPS_OK) return rc;
     const size_t n = (size_t)tot[0];
     if (out_len) *out_len = n;
     if (out_elems) *out_elems = tot[1];
     if (!count_only) {
         if (n > out_cap) return fail(SETOPS_ERR_CAPACITY, "result has %zu elements, output capacity is %zu", n, out_cap);
-        if (n) {
-            HIP_TRY(hipMemcpy(out, dO, n * 4, hipMemcpyDeviceToHost));
-            if (e->bsr) HIP_TRY(hipMemcpy(out_s, dOs, n * 4, hipMemcpyDeviceToHost));
-        }
+        rc = res.get(0, out, n);
+        if (rc == SETOPS_OK && e->bsr) rc = res.get(1, out_s, n);
     }
-    return SETOPS_OK;
+    return rc;
 }
 
+// svs over k > 2 host sets (svs.rs:50-73: the 2-set entry folded over the sets in the given order).
+// Every set is uploaded once, each while the fold before it runs; the intermediate results stay on
+// the device, and a fold waits for the one before it only to know its size.
+int run_svs(int algo, const uint32_t *const *sets, const size_t *lens, size_t k, uint32_t *out, size_t out_cap,
+            size_t *out_len)
+{
+    size_t bytes_in = 0;
+    for (size_t j = 0; j < k; j++) bytes_in += align_up(lens[j] * 4 + 16, 256);
+    const size_t bytes_o = align_up(std::min(lens[0], lens[1]) * 4 + 16, 256);  // bounds every result
+    void *buf = nullptr;
+    int rc = host_scratch(bytes_in + 4 * bytes_o + 256, &buf);
+    if (rc != SETOPS_OK) return rc;
+    hipStream_t s = g_ctx.stream;
+    HostInputs in(static_cast<char *>(buf), bytes_in, false);
+    char *mid = static_cast<char *>(buf) + bytes_in;
+    HostResults res(mid + 2 * bytes_o, bytes_o, 1);
+    const uint32_t *first = in.put(sets[0], lens[0], s, &rc);
+    size_t nfirst = lens[0];
+    const uint32_t *second = in.put(sets[1], lens[1], s, &rc);
+    if (rc == SETOPS_OK) rc = in.send(s);
+    if (rc != SETOPS_OK) return rc;
+    for (size_t j = 1; j < k; j++) {
+        const bool last = j + 1 == k;
+        uint32_t *dst = reinterpret_cast<uint32_t *>(mid + (j & 1) * bytes_o);
+        if (last) dst = out ? res.out[0] : nullptr;
+        rc = single_launch(algo, first, nullptr, nfirst, second, nullptr, lens[j], dst, nullptr,
+                           std::min(nfirst, lens[j]), res.tot, s);
+        if (rc != SETOPS_OK) return rc;
+        unsigned long long tot[2] = {0, 0};
+        rc = res.mark(s);
+        if (rc == SETOPS_OK && !last) {
+            second = in.put(sets[j + 1], lens[j + 1], s, &rc);
+            if (rc == SETOPS_OK) rc = in.send(s);
+        }
+        if (rc == SETOPS_OK) rc = res.wait(s, tot);
+        if (rc != SETOPS_OK) return rc;
+        first = dst;
+        nfirst = (size_t)tot[0];
+    }
+    *out_len = nfirst;
+    if (!out) return SETOPS_OK;
+    if (nfirst > out_cap)
+        return fail(SETOPS_ERR_CAPACITY, "result has %zu elements, output capacity is %zu", nfirst, out_cap);
+    return res.get(0, out, nfirst);
+}
 
 // small_adaptive over k > 2 host sets (adaptive.rs:107-147): every set is uploaded once; one
 // launch intersects the first set with the next one and up to kMaxExtraSets further sets (each
@@ -1040,72 +1199,58 @@ int run_adaptive(int algo, const uint32_t *const *sets, const size_t *lens, size
                  size_t *out_len)
 {
     const size_t groups = (k - 1 + kMaxExtraSets) / (kMaxExtraSets + 1);  // launches of 1 + kMaxExtraSets sets
-    const size_t table = align_up(groups * kMaxExtraSets * 8, 256);      // pointers, then lengths
-    size_t bytes = 256 + 2 * table;
-    for (size_t s = 0; s < k; s++) bytes += align_up(lens[s] * 4 + 16, 256);
+    // a launch's table: kMaxExtraSets pointers, then as many lengths
+    constexpr size_t kTable = 2 * kMaxExtraSets;
+    static_assert(sizeof(void *) == 8, "table words hold pointers");
+    size_t bytes_in = groups * align_up(kTable * 8 + 16, 256);
+    for (size_t j = 0; j < k; j++) bytes_in += align_up(lens[j] * 4 + 16, 256);
     const size_t cap = std::min(lens[0], lens[1]);  // bounds every launch's result
-    const size_t res_bytes = align_up(std::max<size_t>(cap, 1) * 4 + 16, 256);
-    bytes += 2 * res_bytes;
+    const size_t bytes_o = align_up(std::max<size_t>(cap, 1) * 4 + 16, 256);
     void *buf = nullptr;
-    int rc = host_scratch(bytes, &buf);
+    int rc = host_scratch(bytes_in + 4 * bytes_o + 256, &buf);
     if (rc != SETOPS_OK) return rc;
-    char *p = static_cast<char *>(buf);
-    hipStream_t st = g_ctx.stream;
-    unsigned long long *dTot = reinterpret_cast<unsigned long long *>(p);
-    p += 256;
+    hipStream_t s = g_ctx.stream;
+    HostInputs in(static_cast<char *>(buf), bytes_in, false);
+    char *mid = static_cast<char *>(buf) + bytes_in;
+    HostResults res(mid + 2 * bytes_o, bytes_o, 1);
     std::vector<const uint32_t *> dsets(k);
-    for (size_t s = 0; s < k; s++) {
-        uint32_t *d = reinterpret_cast<uint32_t *>(p);
-        if (lens[s]) HIP_TRY(hipMemcpyAsync(d, sets[s], lens[s] * 4, hipMemcpyHostToDevice, st));
-        dsets[s] = d;
-        p += align_up(lens[s] * 4 + 16, 256);
-    }
-    uint32_t *res[2] = {reinterpret_cast<uint32_t *>(p), reinterpret_cast<uint32_t *>(p + res_bytes)};
-    p += 2 * res_bytes;
-    // pointer and length tables of every launch's further sets
-    const uint32_t *const *dX = reinterpret_cast<const uint32_t *const *>(p);
-    p += table;
-    const uint64_t *dL = reinterpret_cast<const uint64_t *>(p);
-    p += table;
+    for (size_t j = 0; j < k; j++) dsets[j] = in.put(sets[j], lens[j], s, &rc);
     // launch g intersects `first` (sets[0], then the previous result) with sets[next] and the
     // further sets sets[next+1 .. next+nx]
+    std::vector<uint64_t> table(groups * kTable, 0);
+    std::vector<const uint32_t *> dtab(groups);
+    for (size_t g = 0; g < groups; g++) {
+        const size_t next = 1 + g * (kMaxExtraSets + 1);
+        for (size_t j = 0; j < (size_t)kMaxExtraSets && next + 1 + j < k; j++) {
+            table[g * kTable + j] = reinterpret_cast<uint64_t>(dsets[next + 1 + j]);
+            table[g * kTable + kMaxExtraSets + j] = lens[next + 1 + j];
+        }
+        dtab[g] = in.put(reinterpret_cast<const uint32_t *>(&table[g * kTable]), 2 * kTable, s, &rc);
+    }
+    if (rc == SETOPS_OK) rc = in.send(s);
+    if (rc != SETOPS_OK) return rc;
     const uint32_t *first = dsets[0];
     size_t nfirst = lens[0];
-    size_t next = 1;
-    int which = 0;
-    for (size_t g = 0; next < k; g++) {
-        if (g >= groups) return fail(SETOPS_ERR_INVALID, "internal: launch count");
-        const size_t nx = std::min<size_t>(kMaxExtraSets, k - next - 1);
-        // the further sets of this launch are sets[next+1 .. next+nx]
-        std::vector<const uint32_t *> gx(kMaxExtraSets, nullptr);
-        std::vector<uint64_t> gl(kMaxExtraSets, 0);
-        for (size_t j = 0; j < nx; j++) {
-            gx[j] = dsets[next + 1 + j];
-            gl[j] = lens[next + 1 + j];
-        }
-        const uint32_t *const *dXg = dX + g * kMaxExtraSets;
-        const uint64_t *dLg = dL + g * kMaxExtraSets;
-        HIP_TRY(hipMemcpyAsync(const_cast<const uint32_t **>(dXg), gx.data(), kMaxExtraSets * sizeof(void *),
-                               hipMemcpyHostToDevice, st));
-        HIP_TRY(hipMemcpyAsync(const_cast<uint64_t *>(dLg), gl.data(), kMaxExtraSets * 8, hipMemcpyHostToDevice, st));
-        rc = single_launch(algo, first, nullptr, nfirst, dsets[next], nullptr, lens[next], res[which], nullptr,
-                           std::max<size_t>(cap, 1), dTot, st, dXg, dLg, (uint32_t)nx);
+    for (size_t g = 0; g < groups; g++) {
+        const size_t next = 1 + g * (kMaxExtraSets + 1);
+        const uint32_t nx = (uint32_t)std::min<size_t>(kMaxExtraSets, k - next - 1);
+        uint32_t *dst = reinterpret_cast<uint32_t *>(mid + (g & 1) * bytes_o);
+        if (g + 1 == groups) dst = out ? res.out[0] : nullptr;
+        rc = single_launch(algo, first, nullptr, nfirst, dsets[next], nullptr, lens[next], dst, nullptr,
+                           std::max<size_t>(cap, 1), res.tot, s, reinterpret_cast<const uint32_t *const *>(dtab[g]),
+                           reinterpret_cast<const uint64_t *>(dtab[g]) + kMaxExtraSets, nx);
         if (rc != SETOPS_OK) return rc;
         unsigned long long tot[2] = {0, 0};
-        HIP_TRY(hipMemcpyAsync(tot, dTot, sizeof tot, hipMemcpyDeviceToHost, st));
-        HIP_TRY(hipStreamSynchronize(st));
-        first = res[which];
+        rc = res.wait(s, tot);
+        if (rc != SETOPS_OK) return rc;
+        first = dst;
         nfirst = (size_t)tot[0];
-        which ^= 1;
-        next += 1 + nx;
     }
     *out_len = nfirst;
-    if (out) {
-        if (nfirst > out_cap)
-            return fail(SETOPS_ERR_CAPACITY, "result has %zu elements, output capacity is %zu", nfirst, out_cap);
-        if (nfirst) HIP_TRY(hipMemcpy(out, first, nfirst * 4, hipMemcpyDeviceToHost));
-    }
-    return SETOPS_OK;
+    if (!out) return SETOPS_OK;
+    if (nfirst > out_cap)
+        return fail(SETOPS_ERR_CAPACITY, "result has %zu elements, output capacity is %zu", nfirst, out_cap);
+    return res.get(0, out, nfirst);
 }
 
 } // namespace
@@ -1240,27 +1385,9 @@ int setops_hip_svs(int algo, const uint32_t *const *sets, const size_t *lens, si
     ENSURE_INIT();
     std::lock_guard<std::mutex> lk(g_ctx.host_mu);
     if (e->kind == KIND_ADAPTIVE && k > 2) return run_adaptive(algo, sets, lens, k, out, out_cap, out_len);
-    // svs.rs:50-73: fold the 2-set entry over the sets in the given order.
-    std::vector<uint32_t> left(std::max<size_t>(1, std::min(lens[0], lens[1]))), right;
-    size_t n = 0;
-    int rc = run_single_pair(algo, sets[0], nullptr, lens[0], sets[1], nullptr, lens[1], left.data(), nullptr,
-                             left.size(), &n, nullptr);
-    if (rc != SETOPS_OK) return rc;
-    for (size_t s = 2; s < k; s++) {
-        std::swap(left, right);
-        left.assign(std::max<size_t>(1, std::min(n, lens[s])), 0u);
-        size_t m = 0;
-        rc = run_single_pair(algo, right.data(), nullptr, n, sets[s], nullptr, lens[s], left.data(), nullptr,
-                             left.size(), &m, nullptr);
-        if (rc != SETOPS_OK) return rc;
-        n = m;
-    }
-    *out_len = n;
-    if (out) {
-        if (n > out_cap) return fail(SETOPS_ERR_CAPACITY, "result has %zu elements, output capacity is %zu", n, out_cap);
-        std::memcpy(out, left.data(), n * 4);
-    }
-    return SETOPS_OK;
+    if (k > 2) return run_svs(algo, sets, lens, k, out, out_cap, out_len);
+    return run_single_pair(algo, sets[0], nullptr, lens[0], sets[1], nullptr, lens[1], out, nullptr, out_cap, out_len,
+                           nullptr);
 }
 
 int setops_hip_intersect2_i32(int algo, const int32_t *a, size_t na, const int32_t *b, size_t nb, int32_t *out,
