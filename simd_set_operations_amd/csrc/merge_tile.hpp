@@ -642,12 +642,18 @@ __global__ __launch_bounds__(NT) void merge_tile_kernel(PairBatch in, TilePlan p
             bstart = boff;
             // A run at key[shift_a ...], B run at key[boff + shift_b ...] (boff = the A run's chunks),
             // loaded straight into LDS; the segment table's loads are in flight meanwhile
+            // The words of many tiles are read once: marked so, they leave the caches to the maps, the
+            // split's lines and the staged results (65,536 uneven pairs with the placement's loads marked
+            // too: 247.5 -> 240.7 us, counted only 40,001 pairs 128.0 -> 124.1, 20,000 balanced ones 199.9 ->
+            // 194.0).  A direct batch is small enough to stay cached (651 balanced pairs: 24.2 us, marked
+            // 25.1).
+            constexpr int kRead = DIRECT ? kLoadKeep : kLoadOnce;
             if (!bad) {
-                stage_run_lds<NT>(in.A, in.a_pool, ga0 & ~3ull, cA, sm.key);
-                stage_run_lds<NT>(in.B, in.b_pool, gb0 & ~3ull, cB, sm.key + boff);
+                stage_run_lds<NT, kRead>(in.A, in.a_pool, ga0 & ~3ull, cA, sm.key);
+                stage_run_lds<NT, kRead>(in.B, in.b_pool, gb0 & ~3ull, cB, sm.key + boff);
                 if constexpr (BSR) {
-                    stage_run_lds<NT>(in.As, in.a_pool, ga0 & ~3ull, cA, sm.st);
-                    stage_run_lds<NT>(in.Bs, in.b_pool, gb0 & ~3ull, cB, sm.st + boff);
+                    stage_run_lds<NT, kRead>(in.As, in.a_pool, ga0 & ~3ull, cA, sm.st);
+                    stage_run_lds<NT, kRead>(in.Bs, in.b_pool, gb0 & ~3ull, cB, sm.st + boff);
                 }
             }
             if (tid < nseg) {

@@ -725,6 +725,11 @@ __global__ __launch_bounds__(NT) void place_tiles_kernel(PairBatch in, TilePlan 
         if (p < pl) return plan.pair_local[p + 1];
         return n + later + (pl + 1 < in.P ? plan.pair_local[pl + 1] : 0u);
     };
+    // staged words are read once; those of many tiles leave the caches to what the stores need
+    auto staged = [](const uint32_t *p) {
+        if constexpr (FUSED) return *p;
+        else return __builtin_nontemporal_load(p);
+    };
     if (out.out) {
         const uint64_t room = out.cap > base ? out.cap - base : 0;
         const uint32_t lim = (uint64_t)n < room ? n : (uint32_t)room;
@@ -737,8 +742,8 @@ __global__ __launch_bounds__(NT) void place_tiles_kernel(PairBatch in, TilePlan 
             for (int j = 0; j < Q; j++) {
                 const uint32_t x = x0 + tid + (uint32_t)j * NT;
                 if (x < lim) {
-                    v[j] = src[x];
-                    if constexpr (BSR) s2[j] = src[sw / 2 + x];
+                    v[j] = staged(src + x);
+                    if constexpr (BSR) s2[j] = staged(src + sw / 2 + x);
                 }
             }
 #pragma unroll
@@ -914,7 +919,9 @@ __device__ __forceinline__ uint4 load_chunk(const uint32_t *__restrict__ src, ui
 // direct global->LDS loads (16 bytes per lane; a wave's row of 64 chunks lands contiguously at
 // the row's LDS address).  The chunk that reaches past the pool (at most the last one) is written
 // element-wise, zero-filled.  The caller waits (s_waitcnt) and synchronizes before reading dst.
-template <int NT>
+// AUX: the loads' cache policy.
+constexpr int kLoadKeep = 0, kLoadOnce = 2;  // (nt: read once, first to leave the caches)
+template <int NT, int AUX>
 __device__ __forceinline__ void stage_run_lds(const uint32_t *__restrict__ src, uint64_t pool, uint64_t base,
                                               uint32_t n, uint32_t *dst)
 {
@@ -923,7 +930,7 @@ __device__ __forceinline__ void stage_run_lds(const uint32_t *__restrict__ src, 
     const uint4 *p = reinterpret_cast<const uint4 *>(src + base);
     const uint32_t lane = threadIdx.x & (kWave - 1);
     for (uint32_t r = threadIdx.x - lane; r < full; r += NT) {  // r: the wave's row (uniform)
-        if (r + lane < full) __builtin_amdgcn_global_load_lds(p + r + lane, dst + 4 * r, 16, 0, 0);
+        if (r + lane < full) __builtin_amdgcn_global_load_lds(p + r + lane, dst + 4 * r, 16, 0, AUX);
     }
     if (full < n && threadIdx.x == 0) {
         const uint64_t e = base + 4ull * full;
