@@ -75,16 +75,20 @@ constexpr int kBsrK = 10;
 constexpr int kKS = kSearchKS[0];
 constexpr int kMaxSeg = 130;
 // gather merge tiles stage every pair's windows as whole 16-byte chunks, so their LDS holds 16
-// words of slack per segment: fewer segments per tile, more tiles per CU (R-MAT scale-22 edges,
-// count-only merge: 587 ms at 130 segments, 490 at 66, 431 at 50 and at 34; the BSR merge, whose
-// tiles hold states too: 600 ms at 50, 526 at 34)
-constexpr int kMaxSegGather = 34;
+// words of slack per segment: fewer segments per tile, more tiles per CU.  The limits are the most
+// that leave six workgroups per CU (LDS is handed out in units of 1,280 bytes): a higher limit pads
+// the pairs less (edge intersections of a scale-16 R-MAT graph, plain merge: 628 us at 26 segments,
+// 610 at 34, 599 at 42, 663 at 58, five per CU; of a scale-17 one with the skew split 1,274, 1,248,
+// 1,228, 1,328; BSR tiles hold states too, their LDS has room for 34)
+constexpr int kMaxSegGather = 42;
+constexpr int kMaxSegGatherBsr = 34;
 // every pair owns at least c0 = ceil(U / (maxseg - 2)) units, so a tile touches at most maxseg
 // pairs; c0 >= K (KS): a lane crosses at most one pair boundary
 constexpr uint32_t pad_for(uint32_t U, int maxseg) { return (U + (maxseg - 2) - 1) / (maxseg - 2); }
 static_assert(pad_for(kNTM * 12, kMaxSeg) >= 12 && pad_for(kNTM * 20, kMaxSeg) >= 20 &&
                   pad_for(kNTM * kBsrK, kMaxSeg) >= kBsrK && pad_for(kNT * 1, kMaxSeg) >= 1 &&
-                  pad_for(kNTM * 12, kMaxSegGather) >= 12 && pad_for(kNTM * 24, kMaxSegGather) >= 24,
+                  pad_for(kNTM * 12, kMaxSegGather) >= 12 && pad_for(kNTM * 24, kMaxSegGather) >= 24 &&
+                  pad_for(kNTM * kBsrK, kMaxSegGatherBsr) >= kBsrK,
               "a lane crosses at most one pair boundary");
 // search policy: words of staged or sampled larger windows per tile (BSR tiles hold states too; both
 // leave the workgroups per CU that the registers allow: four, BSR three)
@@ -300,10 +304,14 @@ uint32_t units_per_tile(Kind k, bool bsr, int shape)
     return merge_like(k) ? (uint32_t)(kNTM * kMergeK[shape]) : (uint32_t)(kNT * kSearchKS[shape]);
 }
 // Segments a tile may touch: gather merge tiles have the smaller limit.
-int max_seg(Kind k, bool gather) { return (gather && merge_like(k)) ? kMaxSegGather : kMaxSeg; }
+int max_seg(Kind k, bool bsr, bool gather)
+{
+    if (!gather || !merge_like(k)) return kMaxSeg;
+    return bsr ? kMaxSegGatherBsr : kMaxSegGather;
+}
 uint32_t pad_units(Kind k, bool bsr, bool gather, int shape)
 {
-    return pad_for(units_per_tile(k, bsr, shape), max_seg(k, gather));
+    return pad_for(units_per_tile(k, bsr, shape), max_seg(k, bsr, gather));
 }
 // Words of one tile's staging slot: keys then (BSR) states, each >= the most results a tile
 // can produce (merge: (U+1)/2 + 1; search: U).
@@ -516,7 +524,7 @@ void launch_merge_t(setops_hip_batch *h, const TileOut &out, hipStream_t stream)
         }
     }
     for (uint64_t t0 = 0; t0 < h->plan.ntiles; t0 += kMaxGrid)
-        hipLaunchKernelGGL((merge_tile_kernel<kNTM, K, GA ? kMaxSegGather : kMaxSeg, BSR, CO, GA, LP>),
+        hipLaunchKernelGGL((merge_tile_kernel<kNTM, K, !GA ? kMaxSeg : BSR ? kMaxSegGatherBsr : kMaxSegGather, BSR, CO, GA, LP>),
                            dim3((uint32_t)std::min<uint64_t>(kMaxGrid, h->plan.ntiles - t0)), dim3(kNTM), 0, stream,
                            h->in, h->plan, out, (uint32_t)t0);
 }
