@@ -55,6 +55,8 @@ def resolve_algo(algo, a_sizes, b_sizes, bsr, indexed=False):
     from . import tuning
 
     best = tuning.choose_resident(a_sizes, b_sizes) if indexed and not bsr else None
+    if best:
+        best = tuning.one_round_shape(best, int(np.minimum(a_sizes, b_sizes).sum()))
     best = best or tuning.choose(a_sizes, b_sizes)
     if bsr:
         from .intersect import registered

@@ -104,6 +104,28 @@ def choose_resident(a_sizes, b_sizes, table=None):
     return min(cost, key=cost.get)
 
 
+# Workgroups of a search tile that run at once: four per CU, of which the dispatcher fills seven in
+# eight (it deals them to the shader engines in turn, and the smallest has 7 of a die's 32 CUs).
+ONE_ROUND_TILES = 896
+# tile shapes of the search entries by probes per lane (SETOPS_SHAPE), fewest first
+SEARCH_SHAPES = ((1, "@1"), (2, ""), (4, "@2"))
+
+
+def one_round_shape(entry, probes):
+    """``entry`` with the fewest probes per lane whose tiles of 256 lanes all run at once: a lane looks
+    its probes up one after another, so where one probe per lane leaves no tile waiting the batch
+    takes one lookup's time (an indexed 2^23-element set against 2,400 probes: 31 us at four probes per
+    lane, 16 at one; against 438,000: 42 at four, 36.5 at two).  Larger batches keep the priced shape, as
+    do other entries."""
+    base, _, _ = entry.partition("@")
+    if base not in ("hip_galloping", "hip_binary_search", "hip_simd_galloping", "hip_small_adaptive"):
+        return entry
+    for k, shape in SEARCH_SHAPES:
+        if probes <= ONE_ROUND_TILES * 256 * k:
+            return base + shape
+    return entry
+
+
 def graph_merge_entry(table=None, default="hip_branchless_merge"):
     """The merge entry (with its tile shape) the autotuner measured fastest for graph edge
     intersections (gather batches over one CSR), or `default` without a measurement."""
