@@ -694,7 +694,7 @@ def main():
         r = {"results": out_total, "info": db.info()}
         for mode in ("out", "count"):
             co = mode == "count"
-            # steps: the run as a caller makes it (a repeated run replays the captured launch graph)
+            # steps: the run as a caller makes it
             for _ in range(3):
                 db.run(stream, count_only=co)
             torch.cuda.synchronize()

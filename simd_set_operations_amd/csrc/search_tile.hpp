@@ -596,12 +596,12 @@ __global__ __launch_bounds__(NT, 4) void search_tile_kernel(PairBatch in, TilePl
         // ---- 3. stage or sample the larger windows while they fit -------------------------------------
         // A window of at most kStage elements per probe is staged whole.  Of a longer one LDS gets
         // the first element of every m-th 128-byte line: at most kSample samples per probe, each
-        // line's read when it is the one that can hold a probe (4a).  So a probe costs at most kSample
+        // line's read when it is the one that can hold a probe (4b).  So a probe costs at most kSample
         // lines of samples (fewer through the index) and one line of the set, in two round trips,
         // where a gallop or binary search from the window's start reads a line per level.  The limits
         // are what LDS holds beside four workgroups per CU.  (3,000 pairs of larger sets of 2^12 to
         // 2^16 elements and ratios up to 4,096: the whole batch 279 us with narrowed windows searched
-        // in global memory, 239 us sampled, 208 us with 4a.)
+        // in global memory, 239 us sampled, 208 us with the staged ones searched as in 4a.)
         uint32_t nst = 0;   // segments whose windows fit
         uint32_t ltot = 0;  // chunks of staged and sampled windows (0: every probe goes through the index)
         constexpr uint32_t kStage = CAPB / U - 1, kSample = CAPB / U > 5 ? 4 : CAPB / U - 1, kMinSample = 24;

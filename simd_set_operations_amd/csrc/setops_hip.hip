@@ -95,7 +95,7 @@ static_assert(pad_for(kNTM * 12, kMaxSeg) >= 12 && pad_for(kNTM * 20, kMaxSeg) >
 constexpr int kCapB = 3584;
 constexpr int kCapBBsr = 2560;
 
-constexpr uint32_t kOneScanGroups = 8;      // pair-unit scans of up to this many groups run as one workgroup
+constexpr uint32_t kOneScanGroups = 8;      // pair-unit scans of up to this many groups run as one kernel
 constexpr uint32_t kOneScanParts = 32;      // ... on at most this many workgroups, each with all the sizes
 constexpr uint32_t kScanDirectGroups = 64;  // tile-count scans of up to this many groups run as one kernel
 constexpr uint64_t kMaxGrid = 1u << 22;  // grid-stride beyond this many workgroups
@@ -465,9 +465,9 @@ int launch_units_scan(setops_hip_batch *h, const TileOut &out, hipStream_t strea
 {
     const uint32_t ng = (uint32_t)((h->P + kScanGroup - 1) / kScanGroup);
     // up to kOneScanGroups groups of pairs (serving steps, small gather batches such as the skewed
-    // workload's 4,096 pairs): the scan is one workgroup, a group at a time
+    // workload's 4,096 pairs): the scan is one kernel of at most kOneScanParts workgroups, each of
+    // which scans the whole batch itself and writes its share of the pairs and tiles
     const bool one = ng <= kOneScanGroups;
-    // (each workgroup scans the batch itself and writes its share of the pairs and tiles)
     const uint32_t parts = grid_for(std::max<uint64_t>(h->P, h->plan.ntiles), kScanGroup);
     if (!one) {
         hipLaunchKernelGGL((units_reduce_kernel<kScanGroup>), dim3(ng), dim3(kScanGroup), 0, stream, h->in,
@@ -692,9 +692,9 @@ int batch_enqueue(setops_hip_batch *h, const TileOut &out, bool count_only, hipS
 // tiles that a fused placement scans) and whether its one tile's outputs are final (plan.one_tile:
 // plain sets, room for every result, the tile's slot is the output).
 //   merge policy: CSR batches and single pairs, whose units have a closed form (601 uneven pairs,
-//     128 tiles: 32 us a run with the plan and split launches, 22.5 us without; a pair of 2^16 + 2^16: 18 and
-//     12 us; beyond the fused placement's tiles the searches in every tile would cost more than
-//     the two launches);
+//     128 tiles: 32 us a run with the plan and split launches, 22.5 us without, both replayed as
+//     graphs, 18.3 us enqueued kernel by kernel; a pair of 2^16 + 2^16: 18 and 12 us; beyond the
+//     fused placement's tiles the searches in every tile would cost more than the two launches);
 //   search policy: gather and CSR batches of at most kNT plain pairs (every tile scans their units),
 //     a single pair of one tile.
 void plan_direct(setops_hip_batch *h, bool count_only, uint64_t cap, bool totals)

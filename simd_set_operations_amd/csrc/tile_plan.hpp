@@ -14,11 +14,13 @@
 // pairs are split across tiles, every tile carries the same work.
 //
 // Pipeline (count -> scan -> write), no communication between workgroups:
-//   plan     unit prefix (closed form for CSR, a three-kernel scan for gather), tile -> pair maps
+//   plan     unit prefix (closed form for CSR, a scan for gather), tile -> pair maps
 //   split    where each tile starts inside its first pair (merge-path split or probe index)
 //   tile     one workgroup per tile: count and stage the tile's results (merge_tile / search_tile)
 //   scan     scan of the tile counts (one kernel when the tiles are few)
 //   place    move staged results to their final positions, per-pair output offsets
+// A run of few tiles has no plan, split or scan launch: its tiles find their own pairs and starts
+// (plan.direct) and the placement sums the tile counts.
 #pragma once
 
 #include "tile_common.hpp"
