@@ -412,7 +412,8 @@ __device__ __forceinline__ void merge_tile_compute(MergeSmem<NT, K, MAXSEG, BSR,
         // nothing (error bit 1) rather than past its slot.
         const uint32_t slot_keys = BSR ? plan.stage_words / 2 : plan.stage_words;
         const uint32_t lds_room = COMPACT ? (nstaged > bstart ? nstaged - bstart : 0u) : ~0u;
-        if (tot > slot_keys || tot > lds_room) {
+        const bool dropped = tot > slot_keys || tot > lds_room;
+        if (dropped) {
             if (tid == 0 && out.error) atomicOr(out.error, 2u);
             tot = 0;
             smask = 0;
@@ -476,6 +477,9 @@ __device__ __forceinline__ void merge_tile_compute(MergeSmem<NT, K, MAXSEG, BSR,
                 el = 0;
                 for (int k = 0; k < NT / kWave; k++) el += sm.wave_el[k];
             }
+            // tile 0 of a direct run clears the error word while other tiles run: the placement
+            // raises the flag again
+            if (DIRECT && dropped && !plan.one_tile) el = kTileDropped;
             plan.tile_count[t] = tot;
             plan.tile_elems[t] = el;
             if (DIRECT && plan.one_tile) {  // its counts are the totals, its results the output

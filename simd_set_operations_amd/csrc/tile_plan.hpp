@@ -630,6 +630,9 @@ __global__ void pair_offsets_kernel(PairBatch in, TilePlan plan, TileOut out)
 // counts before its tile itself and writes its tile's offset, and the workgroup of the last tile
 // writes the totals, the capacity flag and the end offsets.
 constexpr uint32_t kFuseScanTiles = 1024;
+// tile_elems of a direct tile whose results did not fit and were dropped (no tile has so many): the
+// workgroup of the last tile flags it
+constexpr uint32_t kTileDropped = ~0u;
 
 template <int NT, int Q, bool BSR, bool FUSED>
 __global__ __launch_bounds__(NT) void place_tiles_kernel(PairBatch in, TilePlan plan, TileOut out, uint32_t tile0)
@@ -681,7 +684,8 @@ __global__ __launch_bounds__(NT) void place_tiles_kernel(PairBatch in, TilePlan 
                     if (i + j > t && i + j < t2 && i + j < plan.ntiles) later += cw[j];
                     if (last && i + j < plan.ntiles) {
                         const uint32_t ew[4] = {ev[q].x, ev[q].y, ev[q].z, ev[q].w};
-                        el += ew[j];
+                        if (ew[j] != kTileDropped) el += ew[j];
+                        else if (out.error) atomicOr(out.error, 2u);
                     }
                 }
             }
