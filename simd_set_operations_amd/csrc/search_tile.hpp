@@ -19,6 +19,7 @@
 //      tile and per-pair counts -- the same outputs as the merge tile kernel.
 #pragma once
 
+#include "search_window.hpp"
 #include "tile_plan.hpp"
 
 namespace setops {
@@ -606,33 +607,24 @@ __global__ __launch_bounds__(NT, 4) void search_tile_kernel(PairBatch in, TilePl
         uint32_t ltot = 0;  // chunks of staged and sampled windows (0: every probe goes through the index)
         constexpr uint32_t kStage = CAPB / U - 1, kSample = CAPB / U > 5 ? 4 : CAPB / U - 1, kMinSample = 24;
         {
-            uint32_t cl = 0, m = 0, ns = 0, lo = 0, hi = 0;
-            uint64_t gl = 0;
+            LargeWindow lw{};
             uint32_t src = 0;
             bool idx = false;
             if (tid < nseg) {
                 const uint32_t k = sm.seg_wa[tid], f = sm.seg_flags[tid];
+                uint32_t lo = 0, hi = k ? sm.seg_hi[tid] : 0u;
                 idx = through_index((f >> 2) & 1u, sm.seg_hi[tid]);
-                hi = k ? sm.seg_hi[tid] : 0u;
                 if (partial(tid) && (tid == 0 || tid == nseg - 1)) {
                     lo = sm.narrow[tid == 0 ? 0 : 2];
                     hi = sm.narrow[tid == 0 ? 1 : 3];
                 }
-                const uint32_t n = hi - lo;
-                gl = sm.seg_lbase[tid] + lo;
                 src = ((f >> 2) & 1u) ? 0u : 1u;  // pool of the larger side
-                if (idx || n == 0) {
-                    cl = 0;
-                } else if (n <= kStage * k) {
-                    cl = ((uint32_t)(gl & 3) + n + 3) / 4;
-                } else {
-                    const uint32_t heads = (uint32_t)(((gl + n - 1) >> 5) - (gl >> 5));  // lines after the first
-                    const uint32_t most = max(kSample * k, kMinSample);
-                    m = max((heads + most - 1) / most, 1u);
-                    ns = heads / m;
-                    cl = max((ns + 3) / 4, 1u);
-                }
+                const uint64_t base = sm.seg_lbase[tid];
+                if (idx) lw = LargeWindow{base + lo, lo, hi, 0, 0, 0};
+                else lw = large_window(base, lo, hi, k, kStage, kSample, kMinSample);
             }
+            const uint32_t cl = lw.cl, m = lw.m;
+            const uint64_t gl = lw.g;
             const uint32_t lpfx = block_exclusive_scan<NT>(cl, sm.scan_scratch, &ltot);
             const bool fits = lpfx + cl <= (uint32_t)(CAPB / 4);
             // the segments that fit form a prefix; their count is the number of fitting threads
@@ -643,10 +635,10 @@ __global__ __launch_bounds__(NT, 4) void search_tile_kernel(PairBatch in, TilePl
             __syncthreads();
             for (int k = 0; k < NW; k++) nst += sm.wave_el[k];
             if (tid < nseg) {
-                sm.seg_lo[tid] = lo;
-                sm.seg_hi[tid] = hi;
+                sm.seg_lo[tid] = lw.lo;
+                sm.seg_hi[tid] = lw.hi;
                 sm.seg_m[tid] = m;
-                sm.seg_flags[tid] |= ns << 8;
+                sm.seg_flags[tid] |= lw.ns << 8;
                 if (fits) {
                     sm.win_c[tid] = lpfx;
                     sm.win_g[tid] = m ? gl : gl & ~3ull;
