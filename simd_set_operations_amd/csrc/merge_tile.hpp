@@ -418,6 +418,15 @@ __device__ __forceinline__ void merge_tile_compute(MergeSmem<NT, K, MAXSEG, BSR,
             tot = 0;
             smask = 0;
         }
+        // the one tile of a run writes to the caller's output: no further than its capacity (sets have
+        // no more results than that; values repeated in the input may)
+        uint32_t lim = tot;
+        if constexpr (DIRECT && !COUNT_ONLY) {
+            if (plan.one_tile && (uint64_t)tot > out.cap) {
+                lim = (uint32_t)out.cap;
+                if (tid == 0 && out.error) atomicOr(out.error, 1u);
+            }
+        }
         if constexpr (!COUNT_ONLY) {
             uint32_t *dk = plan.stage + (uint64_t)t * plan.stage_words;
             uint32_t *ds = dk + plan.stage_words / 2;
@@ -429,6 +438,7 @@ __device__ __forceinline__ void merge_tile_compute(MergeSmem<NT, K, MAXSEG, BSR,
                     sm_ &= sm_ - 1;
                     const uint32_t ai = (x < nfirst) ? pa0 + x : pa1 + (x - nfirst);
                     const uint32_t v = sm.key[ai];
+                    if (DIRECT && pos >= lim) break;
                     dk[pos] = v;
                     if constexpr (BSR) {
                         // the matching B base lies in the same sub-window: find it again
@@ -466,7 +476,7 @@ __device__ __forceinline__ void merge_tile_compute(MergeSmem<NT, K, MAXSEG, BSR,
                     sm.key[w++] = sm.key[pa0 + __popc(tmask & ((1u << k) - 1u))];
                 }
                 __syncthreads();
-                for (uint32_t i = tid; i < tot; i += NT) dk[i] = sm.key[bstart + i] ^ in_sflip;
+                for (uint32_t i = tid; i < lim; i += NT) dk[i] = sm.key[bstart + i] ^ in_sflip;
             }
         }
 

@@ -45,3 +45,45 @@ def test_dropped_results_are_reported(name, before, after):
                     db.check()
                 assert ei.value.code == _native.SETOPS_ERR_INVALID
         db.close()
+
+
+# one tile whose A repeats values: more results than the output holds, none written past it
+@pytest.mark.parametrize("name,a,b", [
+    ("hip_shuffling", [np.repeat(np.arange(500), 4)], [np.arange(500)]),
+    ("hip_shuffling", [np.repeat(np.arange(100), 4), np.repeat(np.arange(300), 3)], [np.arange(100), np.arange(300)]),
+    ("hip_branchless_merge", [np.full(1004, 5), np.arange(0)], [np.array([5]), np.arange(1000)]),
+])
+def test_one_tile_stays_inside_the_output(name, a, b):
+    import torch
+
+    from simd_set_operations_amd import _native
+    from simd_set_operations_amd.batch import to_device_u32
+    from simd_set_operations_amd.intersect import algo_id
+
+    a, b = ([x.astype(np.uint32) for x in s] for s in (a, b))
+    total, results = sum(x.size for x in a), np.concatenate(a)  # every element of A is found
+    cap = (total + sum(x.size for x in b)) // 2
+    announce(f"one tile {name} {len(a)} pairs, {total} results, room for {cap}")
+    assert total > cap
+    db = csr_batch(name, list(zip(a, b)))
+    assert db.info()["tiles"] == 1
+    lib, stream = _native.hip(), torch.cuda.current_stream().cuda_stream
+    out = torch.full((cap + 4096,), -1, dtype=torch.int32, device="cuda")
+    for _ in range(2):
+        _native.check(lib.setops_hip_batch_run(db.handle, out.data_ptr(), None, cap, db.d_out_off.data_ptr(),
+                                               db.d_counts.data_ptr(), db.d_totals.data_ptr(), stream))
+        with pytest.raises(_native.SetopsError) as ei:
+            db.check()
+        assert ei.value.code == _native.SETOPS_ERR_CAPACITY
+        assert db.totals()[0] == total
+        assert np.array_equal(out[:cap].cpu().numpy().view(np.uint32), results[:cap]) and (out[cap:] == -1).all()
+    db.close()
+    # a single pair has room for the smaller set
+    cap = min(a[0].size, b[0].size)
+    out.fill_(-1)
+    da, d_b = to_device_u32(a[0], torch), to_device_u32(b[0], torch)
+    tot = torch.zeros(2, dtype=torch.int64, device="cuda")
+    _native.check(lib.setops_hip_intersect2_dev(algo_id(name), da.data_ptr(), None, a[0].size, d_b.data_ptr(), None,
+                                                b[0].size, out.data_ptr(), None, cap, tot.data_ptr(), stream))
+    torch.cuda.synchronize()
+    assert (out[cap:] == -1).all()
