@@ -87,3 +87,32 @@ def test_one_tile_stays_inside_the_output(name, a, b):
                                                 b[0].size, out.data_ptr(), None, cap, tot.data_ptr(), stream))
     torch.cuda.synchronize()
     assert (out[cap:] == -1).all()
+
+
+def test_one_search_tile_of_wrong_sizes_stays_inside_the_output():
+    """Device sizes beyond those given to setops_hip_batch_rebind: reported, and written no further than the
+    room that the given sizes ask for."""
+    import torch
+
+    from simd_set_operations_amd import _native
+    from simd_set_operations_amd.batch import GatherBatch
+
+    P = 10
+    pool = np.tile(np.arange(40, dtype=np.uint32), P)
+    beg = np.arange(P, dtype=np.uint64) * np.uint64(40)
+    announce("one search tile, sizes that differ")
+    gb = GatherBatch("hip_galloping", pool, beg, beg + np.uint64(40), pool, beg, beg + np.uint64(40))
+    lib, stream = _native.hip(), torch.cuda.current_stream().cuda_stream
+    one = np.ones(P, np.uint64)
+    _native.check(lib.setops_hip_batch_rebind(gb.handle, gb.dA_beg.data_ptr(), gb.dA_end.data_ptr(),
+                                              gb.dB_beg.data_ptr(), gb.dB_end.data_ptr(), P, one.ctypes.data,
+                                              one.ctypes.data))
+    assert gb.info()["tiles"] == 1
+    out = torch.full((P + 1024,), -1, dtype=torch.int32, device="cuda")
+    _native.check(lib.setops_hip_batch_run(gb.handle, out.data_ptr(), None, P, gb.d_out_off.data_ptr(),
+                                           gb.d_counts.data_ptr(), gb.d_totals.data_ptr(), stream))
+    with pytest.raises(_native.SetopsError) as ei:
+        gb.check()
+    assert ei.value.code == _native.SETOPS_ERR_INVALID and "differ" in str(ei.value)
+    assert (out[P:] == -1).all()
+    gb.close()
