@@ -1164,9 +1164,11 @@ struct HostResults {
         if (g_ctx.pin) std::memcpy(t, g_ctx.pin + kPinIn + kPinOut, 16);
         return SETOPS_OK;
     }
-    // Copies n words of piece i out (after wait).
+    // Copies n words of piece i out (after wait), those that the piece holds: inputs whose values repeat (no
+    // sets) may have more results than there is room for, which no kernel wrote.
     int get(int i, uint32_t *dst, size_t n) const
     {
+        n = std::min(n, step / 4);
         if (!n) return SETOPS_OK;
         if (pinned) std::memcpy(dst, g_ctx.pin + kPinIn + i * step, n * 4);
         else HIP_TRY(hipMemcpy(dst, out[i], n * 4, hipMemcpyDeviceToHost));

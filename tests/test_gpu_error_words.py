@@ -116,3 +116,15 @@ def test_one_search_tile_of_wrong_sizes_stays_inside_the_output():
     assert ei.value.code == _native.SETOPS_ERR_INVALID and "differ" in str(ei.value)
     assert (out[P:] == -1).all()
     gb.close()
+
+
+def test_host_pair_with_repeated_values_copies_only_what_was_written():
+    """A host call whose A repeats values: the count may exceed the smaller set's size, but nothing past the
+    results that the kernels wrote (rounded up to the call's 256-byte pieces) reaches the caller."""
+    from simd_set_operations_amd import intersect
+
+    a, b = np.repeat(np.arange(500, dtype=np.uint32), 4), np.arange(500, dtype=np.uint32)
+    announce("host pair, repeated values")
+    out = np.full(2500, 0xABCD1234, np.uint32)
+    n = intersect.intersect2_c("hip_shuffling", a, b, out)
+    assert n == a.size and np.array_equal(out[:500], a[:500]) and (out[576:] == 0xABCD1234).all()
