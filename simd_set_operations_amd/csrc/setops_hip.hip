@@ -1220,6 +1220,14 @@ int run_single_pair(int algo, const uint32_t *a, const uint32_t *as, size_t na, 
     return rc;
 }
 
+// A fold's result holds at most the smaller set's elements; inputs whose values repeat (no sets) may give
+// more, which the next fold must not read from a buffer made for sets.
+int check_fold(size_t n, size_t na, size_t nb)
+{
+    const size_t cap = std::max<size_t>(1, std::min(na, nb));
+    return n > cap ? fail(SETOPS_ERR_CAPACITY, "result has %zu elements, output capacity is %zu", n, cap) : SETOPS_OK;
+}
+
 // svs over k > 2 host sets (svs.rs:50-73: the 2-set entry folded over the sets in the given order).
 // Every set is uploaded once, each while the fold before it runs; the intermediate results stay on
 // the device, and a fold waits for the one before it only to know its size.
@@ -1255,6 +1263,7 @@ int run_svs(int algo, const uint32_t *const *sets, const size_t *lens, size_t k,
             if (rc == SETOPS_OK) rc = in.send(s);
         }
         if (rc == SETOPS_OK) rc = res.wait(s, tot);
+        if (rc == SETOPS_OK) rc = check_fold((size_t)tot[0], nfirst, lens[j]);
         if (rc != SETOPS_OK) return rc;
         first = dst;
         nfirst = (size_t)tot[0];
@@ -1461,8 +1470,12 @@ int setops_hip_svs(int algo, const uint32_t *const *sets, const size_t *lens, si
     std::lock_guard<std::mutex> lk(g_ctx.host_mu);
     if (e->kind == KIND_ADAPTIVE && k > 2) return run_adaptive(algo, sets, lens, k, out, out_cap, out_len);
     if (k > 2) return run_svs(algo, sets, lens, k, out, out_cap, out_len);
-    return run_single_pair(algo, sets[0], nullptr, lens[0], sets[1], nullptr, lens[1], out, nullptr, out_cap, out_len,
-                           nullptr);
+    size_t n = 0;
+    int rc = run_single_pair(algo, sets[0], nullptr, lens[0], sets[1], nullptr, lens[1], out, nullptr, out_cap, &n,
+                             nullptr);
+    if (int bad = check_fold(n, lens[0], lens[1])) return bad;
+    if (rc == SETOPS_OK || rc == SETOPS_ERR_CAPACITY) *out_len = n;
+    return rc;
 }
 
 int setops_hip_intersect2_i32(int algo, const int32_t *a, size_t na, const int32_t *b, size_t nb, int32_t *out,

@@ -128,3 +128,16 @@ def test_host_pair_with_repeated_values_copies_only_what_was_written():
     out = np.full(2500, 0xABCD1234, np.uint32)
     n = intersect.intersect2_c("hip_shuffling", a, b, out)
     assert n == a.size and np.array_equal(out[:500], a[:500]) and (out[576:] == 0xABCD1234).all()
+
+
+@pytest.mark.parametrize("further", [[], [np.arange(5000)], [np.arange(300), np.arange(5000)]])
+def test_ksets_with_repeated_values_are_refused(further):
+    """A fold that finds more results than its smaller set has elements ends the call with a capacity error,
+    before a further fold reads that many from a buffer of the set's size."""
+    from simd_set_operations_amd import _native, intersect
+
+    sets = [np.repeat(np.arange(500), 4), np.arange(500)] + further
+    announce(f"k-set with repeated values, {len(sets)} sets")
+    with pytest.raises(_native.SetopsError) as ei:
+        intersect.run_kset([s.astype(np.uint32) for s in sets], "hip_shuffling")
+    assert ei.value.code == _native.SETOPS_ERR_CAPACITY
