@@ -710,11 +710,12 @@ __global__ __launch_bounds__(NT, 4) void search_tile_kernel(PairBatch in, TilePl
         // searches in lockstep, so that their reads overlap (two probes, windows of up to 3,000
         // elements: 2,900 cycles where galloping through them in turn takes 6,500)
         if (ltot) {
-            uint32_t at[KS], end[KS], xv[KS], nmax = 0, s = s0;
+            LiftRange r[KS];
+            uint32_t xv[KS], nmax = 0, s = s0;
 #pragma unroll
             for (int k = 0; k < KS; k++) {
                 const uint32_t u = ub + (uint32_t)k;
-                at[k] = end[k] = 1;
+                r[k] = lift_range(0, 0);
                 xv[k] = 0;
                 if (u < ulen) {
                     while (u >= sm.seg_u[s + 1]) s++;
@@ -722,8 +723,7 @@ __global__ __launch_bounds__(NT, 4) void search_tile_kernel(PairBatch in, TilePl
                     if (e < sm.seg_wa[s] && lb != kNotStaged && sm.seg_m[s] == 0) {
                         const uint32_t n = sm.seg_hi[s] - sm.seg_lo[s];
                         xv[k] = sm.pkey[sm.seg_la[s] + e];
-                        at[k] = lb;
-                        end[k] = lb + n;
+                        r[k] = lift_range(lb, n);
                         nmax = max(nmax, n);
                     }
                 }
@@ -732,16 +732,16 @@ __global__ __launch_bounds__(NT, 4) void search_tile_kernel(PairBatch in, TilePl
             for (int bit = (int)L - 1; bit >= 0; bit--) {
 #pragma unroll
                 for (int k = 0; k < KS; k++) {
-                    const uint32_t y = min(at[k] + (1u << bit), end[k]);
+                    const uint32_t y = lift_to(r[k], 1u << bit);
                     // (at its window's end, or without one, a probe stays: y == at)
-                    if (sm.lkey[y - 1] < xv[k]) at[k] = y;
+                    if (sm.lkey[y - 1] < xv[k]) r[k].at = y;
                 }
             }
 #pragma unroll
             for (int k = 0; k < KS; k++) {
-                const bool found = at[k] < end[k] && sm.lkey[at[k]] == xv[k];
+                const bool found = r[k].at < r[k].end && sm.lkey[r[k].at] == xv[k];
                 fmask |= found ? 1u << k : 0u;
-                if constexpr (BSR) lstate[k] = found ? sm.lst[at[k]] : 0u;
+                if constexpr (BSR) lstate[k] = found ? sm.lst[r[k].at] : 0u;
             }
         }
         // 4b. probes of sampled windows, the whole wave together, the k-th probe of every lane at once:

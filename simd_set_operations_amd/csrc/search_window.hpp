@@ -40,4 +40,20 @@ __host__ __device__ __forceinline__ LargeWindow large_window(uint64_t base, uint
     return w;
 }
 
+// The range [at, end) of LDS words that a probe of a staged window of n words from word lb searches.  The
+// lifting reads word y - 1 for at <= y <= end, also where at == end: an empty window, which may begin at
+// word 0, takes the range [1, 1) of a probe without a window.
+struct LiftRange {
+    uint32_t at, end;
+};
+__host__ __device__ __forceinline__ LiftRange lift_range(uint32_t lb, uint32_t n)
+{
+    return n ? LiftRange{lb, lb + n} : LiftRange{1, 1};
+}
+// ... its next position at most `step` further
+__host__ __device__ __forceinline__ uint32_t lift_to(const LiftRange &r, uint32_t step)
+{
+    return r.at + step < r.end ? r.at + step : r.end;
+}
+
 } // namespace setops

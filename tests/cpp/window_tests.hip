@@ -53,9 +53,34 @@ static void windows()
     }
 }
 
+// The words that the lifting reads and the value it finds, over windows anywhere in the staged words, empty ones
+// and the first word included.
+static void lifting()
+{
+    static uint32_t words[4096];
+    for (uint32_t i = 0; i < 4096; i++) words[i] = 3 * i + 1;
+    for (int i = 0; i < 500000; i++) {
+        const uint32_t n = (uint32_t)(rnd(3) ? rnd(40) : rnd(3000)), lb = rnd(3) ? 0u : (uint32_t)rnd(4096 - n);
+        const uint32_t x = (uint32_t)rnd(3 * 4096 + 2), steps = (uint32_t)rnd(13);  // the wave's, at least log2 n
+        setops::LiftRange r = setops::lift_range(lb, n);
+        CHECK(r.at <= r.end && r.end <= 4096, "lb %u n %u", lb, n);
+        uint32_t levels = 0;
+        while (n >> levels) levels++;
+        for (int bit = (int)(steps > levels ? steps : levels) - 1; bit >= 0; bit--) {
+            const uint32_t y = setops::lift_to(r, 1u << bit);
+            CHECK(y >= 1 && y <= 4096, "lb %u n %u: reads word %d", lb, n, (int)y - 1);
+            if (y >= 1 && y <= 4096 && words[y - 1] < x) r.at = y;
+        }
+        uint32_t lower = lb;
+        while (lower < lb + n && words[lower] < x) lower++;
+        CHECK(n == 0 ? r.at == r.end : r.at == lower, "lb %u n %u x %u: %u", lb, n, x, r.at);
+    }
+}
+
 int main()
 {
     windows();
+    lifting();
     std::printf("%d failures\n", failures);
     return failures ? 1 : 0;
 }
