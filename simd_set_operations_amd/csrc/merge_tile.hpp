@@ -614,10 +614,10 @@ __global__ __launch_bounds__(NT) void merge_tile_kernel(PairBatch in, TilePlan p
                 ga1 = edge[1].ga;
                 gb1 = edge[1].gb;
                 edges = TileEdges{edge[0].sa, edge[0].sb, t + 1 < plan.ntiles ? edge[1].pair : ~0u, edge[1].sa, edge[1].sb};
-                if (tid == 0) {  // the maps that the placement reads
-                    plan.tile_first[t] = p_first;
-                    plan.tile_last[t] = p_last;
-                }
+            }
+            if (tid == 0 && !plan.one_tile) {  // the maps that the placement reads
+                plan.tile_first[t] = p_first;
+                plan.tile_last[t] = p_last;
             }
         } else {
             if constexpr (!GATHER) {
