@@ -343,8 +343,10 @@ __global__ __launch_bounds__(NT) void units_scan_kernel(PairBatch in, TilePlan p
         plan.uoff[pb + i] = start[i];
         if (out.counts) out.counts[pb + i] = 0;
     }
-    const bool last = one_group ? part == 0 : pb + n == in.P;
-    if (last && threadIdx.x == 0) plan.uoff[in.P] = start[n];
+    // the pairs scanned include the last one: tiles past the pairs' end (more units planned than the device
+    // sizes make) get pair P here, which the later kernels skip and report
+    const bool last = pb + n == in.P;
+    if (last && part == 0 && threadIdx.x == 0) plan.uoff[in.P] = start[n];
     // the last pair that starts at or before unit v (v >= start[0]; n if the pairs end at or before it)
     auto owner = [&](unsigned long long v) {
         uint32_t lo = 0, hi = n + 1;

@@ -141,3 +141,44 @@ def test_ksets_with_repeated_values_are_refused(further):
     with pytest.raises(_native.SetopsError) as ei:
         intersect.run_kset([s.astype(np.uint32) for s in sets], "hip_shuffling")
     assert ei.value.code == _native.SETOPS_ERR_CAPACITY
+
+
+# pairs in one workgroup's scan, in several workgroups' shares of one, in group scans
+@pytest.mark.parametrize("P", [300, 5000, 9000])
+@pytest.mark.parametrize("name,units", [("hip_galloping", 512), ("hip_branchless_merge", 5120)])
+def test_sizes_beyond_the_device_are_reported(name, units, P):
+    """Host sizes given to setops_hip_batch_rebind that make 3,000 tiles more than the device offsets: the
+    tiles past the pairs' end find no pair, and the run is reported; right sizes then give the results."""
+    from simd_set_operations_amd import _native
+    from simd_set_operations_amd.batch import GatherBatch
+
+    rng = np.random.Generator(np.random.PCG64(P))
+    sets = [np.unique(rng.integers(0, 4000, rng.integers(8, 60))).astype(np.uint32) for _ in range(50)]
+    off = np.concatenate([[0], np.cumsum([s.size for s in sets])]).astype(np.uint64)
+    pool = np.concatenate(sets)
+    ia, ib = rng.integers(0, 50, P), rng.integers(0, 50, P)
+    announce(f"sizes beyond the device {name} P={P}")
+    gb = GatherBatch(name, pool, off[ia], off[ia + 1], pool, off[ib], off[ib + 1])
+    na, nb = (np.ascontiguousarray(off[i + 1] - off[i]) for i in (ia, ib))
+    tiles = gb.info()["tiles"]
+    exp = [np.intersect1d(sets[i], sets[j], assume_unique=True) for i, j in zip(ia, ib)]
+    for more in (3000 * units, 0):
+        hna, hnb = na.copy(), nb.copy()
+        hna[-1] += np.uint64(more)
+        hnb[-1] += np.uint64(more if name == "hip_galloping" else 0)
+        _native.check(_native.hip().setops_hip_batch_rebind(
+            gb.handle, gb.dA_beg.data_ptr(), gb.dA_end.data_ptr(), gb.dB_beg.data_ptr(), gb.dB_end.data_ptr(), P,
+            hna.ctypes.data, hnb.ctypes.data))
+        for rep in range(2):
+            gb.run(count_only=rep == 1)
+            if more:
+                assert gb.info()["tiles"] >= tiles + 2990
+                with pytest.raises(_native.SetopsError) as ei:
+                    gb.check()
+                assert ei.value.code == _native.SETOPS_ERR_INVALID and "differ" in str(ei.value)
+            else:
+                o, cnt, data = gb.results()
+                assert np.array_equal(cnt, [e.size for e in exp])
+                if rep == 0:
+                    assert np.array_equal(data, np.concatenate(exp))
+    gb.close()
