@@ -418,15 +418,10 @@ __device__ __forceinline__ void merge_tile_compute(MergeSmem<NT, K, MAXSEG, BSR,
             tot = 0;
             smask = 0;
         }
-        // the one tile of a run writes to the caller's output: no further than its capacity (sets have
-        // no more results than that; values repeated in the input may)
-        uint32_t lim = tot;
-        if constexpr (DIRECT && !COUNT_ONLY) {
-            if (plan.one_tile && (uint64_t)tot > out.cap) {
-                lim = (uint32_t)out.cap;
-                if (tid == 0 && out.error) atomicOr(out.error, 1u);
-            }
-        }
+        // the one tile of a direct run writes to the caller's output: no further than its capacity (sets
+        // have no more results than that; values repeated in the input may).  Of a run of several tiles
+        // nothing beyond the capacity is placed, so the bound needs no look at the run's form.
+        const uint32_t lim = (DIRECT && !COUNT_ONLY && tot > out.cap) ? (uint32_t)out.cap : tot;
         if constexpr (!COUNT_ONLY) {
             uint32_t *dk = plan.stage + (uint64_t)t * plan.stage_words;
             uint32_t *ds = dk + plan.stage_words / 2;
@@ -487,9 +482,6 @@ __device__ __forceinline__ void merge_tile_compute(MergeSmem<NT, K, MAXSEG, BSR,
                 el = 0;
                 for (int k = 0; k < NT / kWave; k++) el += sm.wave_el[k];
             }
-            // tile 0 of a direct run clears the error word while other tiles run: the placement
-            // raises the flag again
-            if (DIRECT && dropped && !plan.one_tile) el = kTileDropped;
             plan.tile_count[t] = tot;
             plan.tile_elems[t] = el;
             if (DIRECT && plan.one_tile) {  // its counts are the totals, its results the output
@@ -498,6 +490,15 @@ __device__ __forceinline__ void merge_tile_compute(MergeSmem<NT, K, MAXSEG, BSR,
                     out.totals[1] = el;
                 }
                 if (out.out_off) out.out_off[plan.single ? 1 : p_first + nseg] = tot;
+                if (lim < tot && out.error) atomicOr(out.error, 1u);
+            } else if (DIRECT) {
+                // what the placement reads: the maps (stale ones: none, written where they were found) and,
+                // since tile 0 clears the error word while other tiles run, that results were dropped
+                if (nseg) {
+                    plan.tile_first[t] = p_first;
+                    plan.tile_last[t] = p_first + nseg - 1;
+                }
+                if (dropped) plan.tile_elems[t] = kTileDropped;
             }
         }
         if (tid < nseg) {
@@ -614,10 +615,6 @@ __global__ __launch_bounds__(NT) void merge_tile_kernel(PairBatch in, TilePlan p
                 ga1 = edge[1].ga;
                 gb1 = edge[1].gb;
                 edges = TileEdges{edge[0].sa, edge[0].sb, t + 1 < plan.ntiles ? edge[1].pair : ~0u, edge[1].sa, edge[1].sb};
-            }
-            if (tid == 0 && !plan.one_tile) {  // the maps that the placement reads
-                plan.tile_first[t] = p_first;
-                plan.tile_last[t] = p_last;
             }
         } else {
             if constexpr (!GATHER) {

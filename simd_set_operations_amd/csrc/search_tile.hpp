@@ -961,9 +961,10 @@ __global__ __launch_bounds__(NT, 4) void search_tile_kernel(PairBatch in, TilePl
             uint32_t *dk = plan.stage + (uint64_t)t * plan.stage_words;
             uint32_t *ds = dk + plan.stage_words / 2;
             uint32_t pos = pfx2;
-            // the one tile of a run writes to the caller's output: no further than its capacity (device
-            // sizes beyond the planned ones, flagged above, may find more results than it has room for)
-            const uint64_t room = (DIRECT && plan.one_tile) ? out.cap : (uint64_t)U;
+            // the one tile of a direct run writes to the caller's output: no further than its capacity
+            // (device sizes beyond the planned ones, flagged above, may find more results than it has room
+            // for).  Of a run of several tiles nothing beyond the capacity is placed.
+            const uint32_t room = (uint32_t)min(out.cap, (uint64_t)U);
             uint32_t s = s0;
 #pragma unroll
             for (int k = 0; k < KS; k++) {
