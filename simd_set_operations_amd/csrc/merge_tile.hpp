@@ -162,15 +162,19 @@ __device__ __forceinline__ uint32_t block_intersect(const uint32_t *key, const u
     return mask;
 }
 
+// Forms of a tile: planned; direct (plan.direct); direct, a single pair of one tile (merge_pair_kernel).
+enum : int { TF_PLANNED = 0, TF_DIRECT = 1, TF_ONE_PAIR = 2 };
+
 // Steps 3-6 of a tile whose windows and segment table are in LDS (seg_* arrays, key/st): the
 // lanes' merge (or block policy), the tile scan, staged outputs, tile and per-pair counts.
-template <int NT, int K, int MAXSEG, bool BSR, bool COUNT_ONLY, bool GATHER, int LP, bool DIRECT>
+template <int NT, int K, int MAXSEG, bool BSR, bool COUNT_ONLY, bool GATHER, int LP, int FORM>
 __device__ __forceinline__ void merge_tile_compute(MergeSmem<NT, K, MAXSEG, BSR, GATHER, LP != LP_MERGE> &sm,
                                                    const TilePlan &plan, const TileOut &out, uint32_t t,
                                                    uint32_t nseg, uint32_t ulen, uint32_t p_first, uint32_t in_sflip,
                                                    uint32_t nstaged, uint32_t bstart)
 {
     constexpr bool BLOCKP = LP != LP_MERGE;
+    constexpr bool DIRECT = FORM != TF_PLANNED, ONE_PAIR = FORM == TF_ONE_PAIR;
     using Smem = MergeSmem<NT, K, MAXSEG, BSR, GATHER, BLOCKP>;
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = lane_id();
@@ -489,7 +493,7 @@ __device__ __forceinline__ void merge_tile_compute(MergeSmem<NT, K, MAXSEG, BSR,
                     out.totals[0] = tot;
                     out.totals[1] = el;
                 }
-                if (out.out_off) out.out_off[plan.single ? 1 : p_first + nseg] = tot;
+                if (!ONE_PAIR && out.out_off) out.out_off[p_first + nseg] = tot;
                 if (lim < tot && out.error) atomicOr(out.error, 1u);
             } else if (DIRECT) {
                 // what the placement reads: the maps (stale ones: none, written where they were found) and,
@@ -522,8 +526,9 @@ __device__ __forceinline__ void merge_tile_compute(MergeSmem<NT, K, MAXSEG, BSR,
             const uint32_t f = sm.seg_flags[tid];
             const uint64_t p = (uint64_t)p_first + tid;
             if (f & 1u) plan.pair_local[p] = c0v;
-            if (DIRECT && plan.one_tile && out.out_off) out.out_off[p] = c0v;  // every pair lies in the one tile
-            if (out.counts && (!DIRECT || plan.one_tile)) {  // else the placement writes them
+            // (every pair lies in the one tile)
+            if (DIRECT && !ONE_PAIR && plan.one_tile && out.out_off) out.out_off[p] = c0v;
+            if (!ONE_PAIR && out.counts && (!DIRECT || plan.one_tile)) {  // else the placement writes them
                 if ((f & 3u) == 3u) out.counts[p] = c;
                 else if (c) atomicAdd(&out.counts[p], c);
             }
@@ -564,10 +569,11 @@ __device__ __forceinline__ TileStart tile_start(const PairBatch &in, const TileP
 // workgroups.  Each tile's results go to its own staging slot (or nowhere in count-only mode);
 // its counts go to tile_count / tile_elems; per-pair counts and in-tile offsets are recorded for
 // the placement kernel.
-template <int NT, int K, int MAXSEG, bool BSR, bool COUNT_ONLY, bool GATHER, int LP = LP_MERGE, bool DIRECT = false>
-__global__ __launch_bounds__(NT) void merge_tile_kernel(PairBatch in, TilePlan plan, TileOut out, uint32_t tile0)
+template <int NT, int K, int MAXSEG, bool BSR, bool COUNT_ONLY, bool GATHER, int LP, int FORM>
+__device__ __forceinline__ void merge_tile(const PairBatch &in, const TilePlan &plan, const TileOut &out, uint32_t tile0)
 {
     static_assert(K >= 1 && K <= 32, "lane masks hold K bits");
+    constexpr bool DIRECT = FORM != TF_PLANNED, ONE_PAIR = FORM == TF_ONE_PAIR;
     static_assert(!DIRECT || !GATHER, "a direct tile's units have a closed form");
     constexpr int U = NT * K;
     constexpr bool BLOCKP = LP != LP_MERGE;
@@ -587,16 +593,17 @@ __global__ __launch_bounds__(NT) void merge_tile_kernel(PairBatch in, TilePlan p
         // unit, whose units have a closed form, and the merge-path split in it -- two waves find by
         // 64-way searches, five dependent rounds for batches of up to 4,096 pairs; a plan launch and
         // a split launch (a thread per tile, up to 30 dependent loads) cost a small batch 9 us and the
-        // two gaps.  A pair that is one tile starts and ends with it.  A template flag: a runtime
-        // branch here costs the batch tiles 3-5%.
+        // two gaps.  ONE_PAIR: the tile is the pair and finds nothing.  Template flags: a runtime branch
+        // here costs the batch tiles 3-5% and a pair of one tile 0.4 us (300 + 300 elements, calls back to
+        // back: 5.2 us with the branch, 4.8 without).
         constexpr bool direct = DIRECT;
-        __shared__ TileStart edge[DIRECT ? 2 : 1];
+        __shared__ TileStart edge[DIRECT && !ONE_PAIR ? 2 : 1];
         uint64_t ga0 = 0, ga1 = 0, gb0 = 0, gb1 = 0;
         uint32_t p_first = 0, p_last = 0;
         TileEdges edges{};
         if constexpr (direct) {
             if (t == 0 && tid == 0 && out.error) *out.error = 0;  // before thread 0's own flags below
-            if (plan.single && plan.ntiles == 1) {
+            if constexpr (ONE_PAIR) {
                 ga1 = plan.single_na;
                 gb1 = plan.single_nb;
                 edges.next_first = ~0u;
@@ -631,7 +638,7 @@ __global__ __launch_bounds__(NT) void merge_tile_kernel(PairBatch in, TilePlan p
         uint32_t nseg = p_last - p_first + 1;
         bool bad = p_last < p_first || nseg > (uint32_t)MAXSEG || p_last >= in.P;
         if (bad) nseg = 0;
-        if (t == 0 && tid == 0 && out.error && !plan.single &&
+        if (t == 0 && tid == 0 && out.error && !ONE_PAIR && !plan.single &&
             (direct ? in.a_end[in.P - 1] - in.a_beg[0] + in.b_end[in.P - 1] - in.b_beg[0] + (uint64_t)plan.c0 * in.P
                     : plan.uoff[in.P]) != plan.utotal)
             atomicOr(out.error, 4u);
@@ -670,7 +677,7 @@ __global__ __launch_bounds__(NT) void merge_tile_kernel(PairBatch in, TilePlan p
             if (tid < nseg) {
                 if constexpr (direct) {
                     SegRaw r{0, plan.single_na, 0, plan.single_nb, 0, plan.utotal};
-                    if (!plan.single) {
+                    if (!ONE_PAIR && !plan.single) {
                         const uint64_t p = (uint64_t)p_first + tid;
                         r.a = in.a_beg[p];
                         r.a1 = in.a_end[p];
@@ -680,7 +687,7 @@ __global__ __launch_bounds__(NT) void merge_tile_kernel(PairBatch in, TilePlan p
                         r.u1 = r.u + (r.a1 - r.a) + (r.b1 - r.b) + plan.c0;
                     }
                     w = seg_window(plan, r, t, p_first, nseg, tid, ulen, edges);
-                    if (w.flags & 1u) plan.uoff[(uint64_t)p_first + tid] = r.u;  // for the placement
+                    if (!ONE_PAIR && (w.flags & 1u)) plan.uoff[(uint64_t)p_first + tid] = r.u;  // for the placement
                 } else {
                     w = seg_window(in, plan, t, p_first, nseg, tid, ulen);
                 }
@@ -752,9 +759,22 @@ __global__ __launch_bounds__(NT) void merge_tile_kernel(PairBatch in, TilePlan p
             }
         }
 
-        merge_tile_compute<NT, K, MAXSEG, BSR, COUNT_ONLY, GATHER, LP, DIRECT>(sm, plan, out, t, nseg, ulen, p_first,
+        merge_tile_compute<NT, K, MAXSEG, BSR, COUNT_ONLY, GATHER, LP, FORM>(sm, plan, out, t, nseg, ulen, p_first,
                                                                        in.sflip, staged_words, bstart);
     }
+}
+
+template <int NT, int K, int MAXSEG, bool BSR, bool COUNT_ONLY, bool GATHER, int LP = LP_MERGE, bool DIRECT = false>
+__global__ __launch_bounds__(NT) void merge_tile_kernel(PairBatch in, TilePlan plan, TileOut out, uint32_t tile0)
+{
+    merge_tile<NT, K, MAXSEG, BSR, COUNT_ONLY, GATHER, LP, DIRECT ? TF_DIRECT : TF_PLANNED>(in, plan, out, tile0);
+}
+
+// A single pair of one tile (no per-pair offsets and counts).
+template <int NT, int K, int MAXSEG, bool BSR, bool COUNT_ONLY, int LP>
+__global__ __launch_bounds__(NT) void merge_pair_kernel(PairBatch in, TilePlan plan, TileOut out)
+{
+    merge_tile<NT, K, MAXSEG, BSR, COUNT_ONLY, false, LP, TF_ONE_PAIR>(in, plan, out, 0u);
 }
 
 } // namespace setops

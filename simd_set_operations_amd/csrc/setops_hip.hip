@@ -518,8 +518,12 @@ void launch_merge_t(setops_hip_batch *h, const TileOut &out, hipStream_t stream)
 {
     if constexpr (!GA) {
         if (h->plan.direct) {
-            hipLaunchKernelGGL((merge_tile_kernel<kNTM, K, kMaxSeg, BSR, CO, GA, LP, true>),
-                               dim3((uint32_t)h->plan.ntiles), dim3(kNTM), 0, stream, h->in, h->plan, out, 0u);
+            if (h->plan.single && h->plan.ntiles == 1)
+                hipLaunchKernelGGL((merge_pair_kernel<kNTM, K, kMaxSeg, BSR, CO, LP>), dim3(1), dim3(kNTM), 0, stream,
+                                   h->in, h->plan, out);
+            else
+                hipLaunchKernelGGL((merge_tile_kernel<kNTM, K, kMaxSeg, BSR, CO, GA, LP, true>),
+                                   dim3((uint32_t)h->plan.ntiles), dim3(kNTM), 0, stream, h->in, h->plan, out, 0u);
             return;
         }
     }
