@@ -495,14 +495,11 @@ __device__ __forceinline__ void merge_tile_compute(MergeSmem<NT, K, MAXSEG, BSR,
                 }
                 if (!ONE_PAIR && out.out_off) out.out_off[p_first + nseg] = tot;
                 if (lim < tot && out.error) atomicOr(out.error, 1u);
-            } else if (DIRECT) {
-                // what the placement reads: the maps (stale ones: none, written where they were found) and,
-                // since tile 0 clears the error word while other tiles run, that results were dropped
-                if (nseg) {
-                    plan.tile_first[t] = p_first;
-                    plan.tile_last[t] = p_first + nseg - 1;
-                }
-                if (dropped) plan.tile_elems[t] = kTileDropped;
+            } else if (DIRECT && nseg && (ONE_PAIR || dropped)) {
+                // the maps that the placement reads, or that results were dropped (tile 0 clears the error
+                // word while other tiles run): the placement then raises the flag again
+                plan.tile_first[t] = p_first;
+                plan.tile_last[t] = dropped ? ~(p_first + nseg - 1) : p_first + nseg - 1;
             }
         }
         if (tid < nseg) {
@@ -622,6 +619,10 @@ __device__ __forceinline__ void merge_tile(const PairBatch &in, const TilePlan &
                 ga1 = edge[1].ga;
                 gb1 = edge[1].gb;
                 edges = TileEdges{edge[0].sa, edge[0].sb, t + 1 < plan.ntiles ? edge[1].pair : ~0u, edge[1].sa, edge[1].sb};
+                if (tid == 0) {  // the maps that the placement reads
+                    plan.tile_first[t] = p_first;
+                    plan.tile_last[t] = p_last;
+                }
             }
         } else {
             if constexpr (!GATHER) {

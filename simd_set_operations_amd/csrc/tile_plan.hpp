@@ -632,9 +632,6 @@ __global__ void pair_offsets_kernel(PairBatch in, TilePlan plan, TileOut out)
 // counts before its tile itself and writes its tile's offset, and the workgroup of the last tile
 // writes the totals, the capacity flag and the end offsets.
 constexpr uint32_t kFuseScanTiles = 1024;
-// tile_elems of a direct tile whose results did not fit and were dropped (no tile has so many): the
-// workgroup of the last tile flags it
-constexpr uint32_t kTileDropped = ~0u;
 
 template <int NT, int Q, bool BSR, bool FUSED>
 __global__ __launch_bounds__(NT) void place_tiles_kernel(PairBatch in, TilePlan plan, TileOut out, uint32_t tile0)
@@ -646,10 +643,14 @@ __global__ __launch_bounds__(NT) void place_tiles_kernel(PairBatch in, TilePlan 
     const uint64_t pf = plan.tile_first[t];
     uint64_t pl = plan.tile_last[t];
     if (pl >= in.P) {
-        // stale maps (flagged by the tile kernel; the tiles of a direct plan, which race with the one
-        // that clears the flags, leave it to this kernel): stay inside the pairs
-        if (FUSED && plan.direct && tid == 0 && out.error) atomicOr(out.error, 2u);
+        // stale maps (flagged by the tile kernel): stay inside the pairs.  The tiles of a direct plan, which
+        // race with the one that clears the flags, leave the flag to this kernel: one without pairs, and
+        // one that dropped its results, which holds the complement of its last pair.
         pl = in.P - 1;
+        if (FUSED && plan.direct) {
+            pl = min(pl, (uint64_t)~plan.tile_last[t]);
+            if (tid == 0 && out.error) atomicOr(out.error, 2u);
+        }
     }
     uint64_t base;
     uint32_t n;
@@ -686,8 +687,7 @@ __global__ __launch_bounds__(NT) void place_tiles_kernel(PairBatch in, TilePlan 
                     if (i + j > t && i + j < t2 && i + j < plan.ntiles) later += cw[j];
                     if (last && i + j < plan.ntiles) {
                         const uint32_t ew[4] = {ev[q].x, ev[q].y, ev[q].z, ev[q].w};
-                        if (ew[j] != kTileDropped) el += ew[j];
-                        else if (out.error) atomicOr(out.error, 2u);
+                        el += ew[j];
                     }
                 }
             }
