@@ -6,7 +6,7 @@ Grid: larger-set size 2^6 .. 2^14, skew (larger / smaller) 2^0 .. 2^10, selectiv
 0.9, density 0.1 (element space = 10 x larger), the planted-shared-then-disjoint data of the
 benchmark workloads.  Each cell is a fixed-shape CSR batch of about 2^26 input elements (at most
 2^18 pairs); every entry runs it as a device batch (plan, tile kernel, scan, placement, with
-outputs) and is timed over replayed runs with HIP events, after a check of its per-pair counts
+outputs) and is timed over repeated runs with HIP events, after a check of its per-pair counts
 against the planted counts.  The table (``tuning.json``) feeds :mod:`.tuning`, which prices a
 batch per entry and picks the cheapest (``hip_auto``).  It also holds the search entries' probe
 rates against one indexed resident set (the skewed workload's shape, per smaller-set size).
@@ -123,7 +123,7 @@ RESIDENT_ALGOS = ("hip_galloping", "hip_galloping@1", "hip_galloping@2", "hip_bi
 def resident_cells(torch, runs=5, log=print, log2_small=RESIDENT_LOG2_SMALL, algos=RESIDENT_ALGOS):
     """Probes per second of the search entries against one indexed resident set, per smaller-set
     size: GatherBatch(..., index=True) over the skewed workload's large set, counts checked against
-    the planted ones, replayed runs timed with HIP events."""
+    the planted ones, repeated runs timed with HIP events."""
     from . import datagen
     from .batch import GatherBatch
 

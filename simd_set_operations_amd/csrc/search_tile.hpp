@@ -11,10 +11,12 @@
 //      partition search,
 //   3. stage the larger windows in LDS, whole where they are short, else the first element of every
 //      m-th line, while they fit (a prefix of the segments); the rest are searched in global memory,
-//   4. each lane looks up its KS probes, in sampled windows by groups of lanes that read the line
-//      found, in staged and unstaged ones in order, from where the previous probe landed: galloping (exponential then binary, galloping.rs:7-30), binary search over the rest of
-//      the window (binary_search_intersect, galloping.rs:32-49) or block galloping with a full
-//      compare of the last block (simd_galloping.rs:49-107),
+//   4. each lane looks up its KS probes: in windows staged whole by binary lifting, in sampled windows
+//      and through the B-pool index by groups of lanes that read the line found, the same for every
+//      entry.  The search mode tells the entries apart where a window found no room (and for further
+//      sets): galloping (exponential then binary, galloping.rs:7-30), binary search
+//      (binary_search_intersect, galloping.rs:32-49) or block galloping with a full compare of the
+//      last block (simd_galloping.rs:49-107), each probe from the window's start,
 //   5. block scan of hits, results (probe values; BSR: base and state AND) staged in order,
 //      tile and per-pair counts -- the same outputs as the merge tile kernel.
 #pragma once

@@ -460,7 +460,7 @@ uint32_t grid_for(uint64_t n, uint64_t per_block)
     return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(g, kMaxGrid));
 }
 
-// Unit prefix by the three-kernel scan (gather batches, search policy).
+// Unit prefix by a scan of the pairs' units (gather batches, search policy): one kernel or three.
 int launch_units_scan(setops_hip_batch *h, const TileOut &out, hipStream_t stream)
 {
     const uint32_t ng = (uint32_t)((h->P + kScanGroup - 1) / kScanGroup);
@@ -919,10 +919,10 @@ int single_launch(int algo, const uint32_t *dA, const uint32_t *dAs, size_t na, 
 }
 
 // setops_hip_intersect2_dev_noalloc: one pair planned and staged in the device scratch array.  The
-// launch sequence is single_launch's, enqueued eagerly (no graph capture, no events), and nothing
-// is allocated: the workspace and the staging slots are laid out in the scratch of the current
-// device.  Every pipeline kernel writes what a later one reads (the plan kernel clears the totals,
-// the error word and the counts), so the scratch needs no clearing between calls.
+// launch sequence is single_launch's, without events, and nothing is allocated: the workspace and
+// the staging slots are laid out in the scratch of the current device.  Every pipeline kernel writes
+// what a later one reads (the plan kernel, or a direct run's tiles, clear or write the totals, the
+// error word and the maps), so the scratch needs no clearing between calls.
 constexpr uint64_t kNoAllocMaxMerge = 1ull << 22;   // na + nb of a merge-path entry
 constexpr uint64_t kNoAllocMaxProbes = 1ull << 20;  // min(na, nb) of a search entry
 setops_hip_batch g_noalloc;  // the call's host-side description (reused; owns no device memory)
@@ -1000,8 +1000,11 @@ int noalloc_launch(int algo, const uint32_t *dA, const uint32_t *dAs, size_t na,
 // into that memory, so that a call waits once, for its kernels, and copies its result out.  (A copy of
 // the runtime costs 8 to 15 us, whatever its size: with two uploads, the totals and the result a pair
 // of 1,000 + 1,300 took 50 us, 24 now; a k-set query of 5 sets of up to 2^18, 16 copies, 311 us, 171
-// now.  Up to kMapIn the copy kernel costs more than reading over the bus: 84 KB 33 against 30.5 us, 107
-// KB 33.5 against 33.8.)  Larger inputs and results go by the runtime's copies.
+// now.  Up to kMapIn a merge entry reads over the bus in less time than the copy kernel takes: 1,000
+// + 1,300 elements 22.3 against 25 us, 84 KB 30.5 against 33, 107 KB 33.8 against 33.5.  A search entry, whose
+// reads depend on one another, breaks even at about 24 KB: 100 + 100 elements 25.6 against 26.6 us, 200 +
+// 20,000 34.5 against 34.3, but 1,000 + 20,000 43 against 40.5 and 20 + 20,000 39.8 against 35.5; with
+// copies of the runtime they took 72 to 96.)  Larger inputs and results go by the runtime's copies.
 constexpr size_t kMapIn = 96u << 10;
 constexpr size_t kPinIn = 4u << 20;
 constexpr size_t kPinOut = 2u << 20;

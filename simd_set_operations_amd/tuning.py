@@ -112,11 +112,14 @@ SEARCH_SHAPES = ((1, "@1"), (2, ""), (4, "@2"))
 
 
 def one_round_shape(entry, probes):
-    """``entry`` with the fewest probes per lane whose tiles of 256 lanes all run at once: a lane looks
-    its probes up one after another, so where one probe per lane leaves no tile waiting the batch
-    takes one lookup's time (an indexed 2^23-element set against 2,400 probes: 31 us at four probes per
-    lane, 16 at one; against 438,000: 42 at four, 36.5 at two).  Larger batches keep the priced shape, as
-    do other entries."""
+    """``entry`` with the fewest probes per lane whose probes fill tiles of 256 lanes that all run at once: a
+    lane looks its probes up one after another, so where one probe per lane leaves no tile waiting the
+    batch takes one lookup's time (an indexed 2^23-element set against 2,400 probes: 31 us at four probes
+    per lane, 16 at one; against 438,000: 42 at four, 36.5 at two).  Larger batches keep the priced shape,
+    as do other entries.  Sets too small for a tile's pair limit (under 2, 4 or 8 probes) are padded by
+    that many units each, so that batches of them run in up to three rounds; the shape is still faster
+    than the priced one (200,000 sets of one element, 2,344 tiles at one probe per lane: 57.5 us, 63.1 at
+    two, 82.2 at four; 100,000 of them 43.7, 40.4, 52.8; 100,000 of two 35.1, 55.3, 53.5)."""
     base, _, _ = entry.partition("@")
     if base not in ("hip_galloping", "hip_binary_search", "hip_simd_galloping", "hip_small_adaptive"):
         return entry
