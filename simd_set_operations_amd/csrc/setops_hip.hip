@@ -512,7 +512,8 @@ int device_unit_total(setops_hip_batch *h, uint64_t *utotal, uint64_t *small)
 
 // Tile kernels run one workgroup per tile; batches of more than kMaxGrid tiles take several
 // launches (tile offset tile0).  A direct plan launches the kernels' DIRECT form, which finds its
-// tiles' pairs itself instead of reading the tile maps.
+// tiles' pairs itself instead of reading the tile maps, or, for a single pair of one merge tile, the
+// pair's own kernel.
 template <int K, bool BSR, bool CO, bool GA, int LP>
 void launch_merge_t(setops_hip_batch *h, const TileOut &out, hipStream_t stream)
 {
